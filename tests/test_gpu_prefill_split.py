@@ -1,0 +1,138 @@
+"""The prefill GEMM's plans at their edges, in the exact-integer mode (every scale 1, so that any order
+of the sums gives the same output): K split over workgroups (the torch ops, whose workspace has room
+for the parts) and unsplit (gguf_mul_mat with the workspace gguf_op_workspace_bytes asks for), for
+every type it serves, at row counts that are no multiple of a 128-row tile and activation rows at the
+edges of its 64-, 128- and 256-column tiles; graph replays of a split product; Q6_K's two-plane
+operands at the largest sub-scales; the no-allocation entry point in parts. Needs an MI355X.
+"""
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import gguf_oracle as o
+from _gpu import C, dev, exact_ref, exact_weights, exact_x, graph_replays_equal, w_rand, x_rand
+
+pytestmark = pytest.mark.gpu
+
+PACKED = (o.IQ3_S, o.IQ3_XXS)
+TYPES = [o.IQ3_S, o.IQ3_XXS, o.Q4_K, o.Q6_K, o.IQ4_XS, o.Q2_K, o.IQ2_XXS, o.IQ2_XS, o.IQ2_S]
+MUL_MAT_Q, PACKED_TILED = 1, 7
+
+
+@pytest.fixture(scope="module")
+def lib():
+    assert torch.cuda.is_available(), "GPU tests need an MI355X"
+    from vllm_gguf_plugin import _capi, ops  # noqa: F401
+
+    return _capi.load()
+
+
+def _weight(qt, raw):
+    from vllm_gguf_plugin.quantization import iq3_pack
+
+    return iq3_pack.pack(dev(raw), qt) if qt in PACKED else dev(raw)
+
+
+def _torch_op(qt, w, x, rows):
+    op = "lcpp_mul_mat_iq3_packed" if qt in PACKED else "lcpp_mul_mat_q"
+    return getattr(C(), op)(w, x, qt, rows)
+
+
+def _capi_op(lib, qt, w, x, rows, entry="workspace"):
+    from vllm_gguf_plugin import _capi
+
+    op, (n, k) = (PACKED_TILED if qt in PACKED else MUL_MAT_Q), x.shape
+    y = torch.full((n, rows), float("nan"), dtype=x.dtype, device="cuda")
+    nb = lib.gguf_op_workspace_bytes(op, qt, rows, k, n, 0)
+    stream = torch.cuda.current_stream().cuda_stream
+    args = (op, _capi.ref(_capi.view(w)), _capi.ref(_capi.view(x)), qt, rows, None, y.data_ptr(), y.numel() * y.element_size())
+    if entry == "noalloc":
+        rc = lib.gguf_mul_mat_noalloc(*args, stream)
+    else:
+        ws = torch.full((max(nb, 1),), 0xFF, dtype=torch.uint8, device="cuda")
+        rc = lib.gguf_mul_mat(*args, ws.data_ptr(), nb, stream)
+    assert rc == 0, _capi.error(lib)
+    torch.cuda.synchronize()
+    return y, nb
+
+
+# rows (packed types: the next multiple of 16), K, activation rows: two row tiles and a ragged third, K
+# blocks that the runs cut unevenly; one 16-row tile; K of one step pair
+SHAPES = [(270, 4608, 257), (270, 4608, 300), (16, 1024, 513), (1030, 512, 259), (130, 2560, 1025)]
+
+
+@pytest.mark.parametrize("rows,k,n", SHAPES)
+@pytest.mark.parametrize("qt", TYPES, ids=lambda t: o.TYPE_NAMES[t])
+def test_split_and_unsplit_exact(lib, qt, rows, k, n):
+    rows = -(-rows // 16) * 16 if qt in PACKED else rows
+    raw = exact_weights(qt, rows, k, seed=rows + n)
+    x = exact_x(n, k, seed=n, dtype=torch.float32)
+    ref = exact_ref(raw, qt, x, form="mmq")
+    w, xg = _weight(qt, raw), x.cuda()
+    assert np.array_equal(_torch_op(qt, w, xg, rows).cpu().numpy(), ref)
+    y, nb = _capi_op(lib, qt, w, xg, rows)
+    assert nb == -(-n // 16) * (k // 256) * (8192 + (2048 if qt == o.Q2_K else 1024))  # the prefill GEMM's layout
+    assert np.array_equal(y.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("n", [1, 8, 16, 17, 63, 64, 65, 128, 129])
+def test_q2k_every_row_count(n):
+    """Q2_K's product op runs the prefill GEMM at any row count: 64-column tiles (four row parts)."""
+    raw = exact_weights(o.Q2_K, 270, 2560, seed=n)
+    x = exact_x(n, 2560, seed=n + 1, dtype=torch.float32)
+    y = _torch_op(o.Q2_K, dev(raw), x.cuda(), 270).cpu().numpy()
+    assert np.array_equal(y, exact_ref(raw, o.Q2_K, x, form="mmq"))
+
+
+@pytest.mark.parametrize("qt", [o.Q4_K, o.IQ4_XS, o.Q6_K, o.IQ2_S], ids=lambda t: o.TYPE_NAMES[t])
+@pytest.mark.parametrize("n", [33, 49, 64])
+def test_rows_33_to_64(qt, n):
+    """Weights of 24M values or more at 33..64 rows: the torch ops prefer the prefill GEMM there (64
+    columns per workgroup, K split). fp32 X against the q81 model on sampled rows."""
+    rows, k = 5120, 5120
+    raw = w_rand(qt, rows, k, seed=n)
+    x = x_rand(n, k, seed=n + 7)
+    rs = np.unique(np.random.default_rng(n).choice(rows, 48, replace=False))
+    y = _torch_op(qt, dev(raw), x.cuda(), rows).cpu().numpy()[:, rs]
+    assert o.rel_l2(y, o.q81_model(raw[rs], qt, x, layout="mmq")) <= 1e-3
+
+
+def test_split_graph_replays():
+    """Replays of a captured split product (its counters are cleared by the captured quantise launch),
+    with eager work between, equal the eager result bit for bit."""
+    raw = w_rand(o.Q4_K, 1030, 2560, seed=1)
+    w, x = dev(raw), x_rand(300, 2560, seed=2, dtype=torch.bfloat16).cuda()
+    eager = _torch_op(o.Q4_K, w, x, 1030)
+    assert torch.equal(eager, _torch_op(o.Q4_K, w, x, 1030))
+    graph_replays_equal(lambda: torch.ops._C_gguf.lcpp_mul_mat_q(w, x, o.Q4_K, 1030), eager)
+
+
+def test_q6k_two_planes_largest_subscales():
+    """Q6_K below the rounded plan's rows: every sub-scale +-127 or -128, products up to 4096 kept
+    exact in two operand planes (the int8 GEMM's results)."""
+    rows, k, n = 270, 2560, 259
+    raw = exact_weights(o.Q6_K, rows, k, seed=3)
+    sc = np.random.default_rng(4).choice(np.array([127, -127, -128], np.int8), size=(rows * k // 256, 16))
+    raw.reshape(-1, 210)[:, 192:208] = sc.view(np.uint8)
+    x = exact_x(n, k, seed=5, dtype=torch.float32)
+    y = _torch_op(o.Q6_K, dev(raw), x.cuda(), rows).cpu().numpy()
+    ref = exact_ref(raw, o.Q6_K, x, form="mmq")
+    # integers below 2^24 (exact_ref asserts it): any order of the fp32 sums is exact
+    assert np.array_equal(y, ref)
+
+
+@pytest.mark.parametrize("qt,n", [(o.IQ4_XS, 1100), (o.IQ2_S, 1100), (o.Q2_K, 900)], ids=["IQ4_XS", "IQ2_S", "Q2_K"])
+def test_noalloc_in_parts(lib, qt, n):
+    """Products whose fp16 activation copy exceeds the static scratch and whose int8 copy fits it: the
+    no-allocation entry point runs them in parts of the activation rows, with the same results."""
+    rows, k = 400, 5120
+    w = dev(w_rand(qt, rows, k, seed=n))
+    x = x_rand(n, k, seed=n + 1, dtype=torch.float32).cuda()
+    a, need = _capi_op(lib, qt, w, x, rows, "noalloc")
+    assert need > lib.gguf_scratch_bytes()
+    b, _ = _capi_op(lib, qt, w, x, rows)
+    # the parts' plans may add in another order: 8 fp32 roundings of sums of 160 slice terms
+    assert float((a - b).norm() / b.norm()) <= 8 * 2.0 ** -24 * np.sqrt(160)

@@ -54,14 +54,16 @@ hipError_t launch_gemv_generic_x(int type, const uint8_t* W, int64_t row_bytes, 
 hipError_t launch_gemm_packed_xq(const uint8_t* W, int64_t row_bytes, int nrows, int k, const uint8_t* xq, int n,
                                  void* y, int y_dtype, void* split_ws, hipStream_t stream);
 hipError_t launch_quantize_xh(const void* x, int dtype, int64_t n, int64_t k, int64_t s01, int type, void* y,
-                              hipStream_t stream);
-bool prefill_uses_xh(int type, bool packed);
+                              hipStream_t stream, uint32_t* zero = nullptr, int64_t zero_words = 0);
+bool prefill_supported(int type, bool packed);
+int64_t prefill_counters(int64_t nrows, int64_t k, int64_t n);
+size_t prefill_slot_bytes(int64_t nrows, int64_t k, int64_t n);
 bool small_h_supported(int type, bool packed);
 bool small_h_range(int type, int64_t nrows, int64_t n);
 hipError_t launch_gemm_small_h(int type, bool packed, const uint8_t* W, int64_t row_bytes, int nrows, int k,
                                const uint8_t* xh, int n, void* y, int y_dtype, hipStream_t stream);
-hipError_t launch_gemm_prefill(int type, bool packed, const uint8_t* W, int64_t row_bytes, int nrows, int k,
-                               const uint8_t* xq, int n, void* y, int y_dtype, hipStream_t stream);
+hipError_t launch_gemm_prefill(int type, bool exact, const uint8_t* W, int64_t row_bytes, int nrows, int k, const uint8_t* xh, int n,
+                               void* y, int y_dtype, float* part, uint32_t* cnt, hipStream_t stream);
 hipError_t launch_iq3_pack(int type, uint8_t* w, int64_t rows, int64_t row_bytes, bool unpack, uint8_t* scratch,
                            size_t scratch_bytes, hipStream_t stream);
 size_t iq3_pack_scratch_bytes(int64_t rows, int64_t row_bytes);
@@ -70,6 +72,9 @@ hipError_t launch_dense(int dtype, const void* W, int64_t ws0, int rows, int k, 
 }  // namespace gguf
 
 namespace {
+
+// the no-allocation entry point's static workspace
+constexpr size_t kScratchBytes = GGUF_SCRATCH_BYTES;
 
 thread_local std::string g_err;
 
@@ -257,33 +262,52 @@ bool packed_fused(int op, int64_t row, int64_t k, int64_t n, bool has_x_q8) {
 // inside the GEMV at one or two rows where each wave's part of X is small (K <= 8192).
 bool rows_fused(int op, int64_t type, int64_t row, int64_t k, int64_t n, bool has_x_q8);
 
-// Product ops go to the 128 x 128-tile prefill GEMM from this many activation rows on (the small
-// GEMMs' one-column-tile-group plans re-decode the weights once per 16..64 activation rows).
-constexpr int64_t kPrefillFrom = 256;
-
 bool xxs_packed(int op, int64_t type);
 
-// Whether a product op runs the prefill GEMM (128 weight rows x 256 activation rows per
-// workgroup; 128 on grids of fewer than 256). Its grid must hold enough workgroups: per
-// workgroup it walks all of K, so on a small grid most CUs idle while the small GEMMs (16-row
-// tiles) spread the same work. Measured (µs per op, graph replays, prefill / small GEMM):
-//   1024 x 5120, M = 256 / 512 (8 / 16 groups): IQ3_S 106 / 109 against 26 / 38, Q6_K 113 / 114
-//   against 28 / 49; M = 2048 (64 groups): IQ3_S 124 against 134, Q6_K 127 against 166;
-//   6144 x 5120, M = 256 (48): IQ3_S 108 against 95, Q4_K 117 against 96; M = 512 (96): 114
-//   against 168, 123 against 184; 5120 x 17408, M = 256 (40): IQ3_S 314 against 224; M = 512
-//   (80): 323 against 430; 17408 x 5120, M = 256 (136): 152 against 158.
-// So from 64 groups on (128 for IQ4_XS, whose prefill GEMM is the int8 one: 5120 x 6144 M = 512,
-// 80 groups, 219 against 182; 17408 x 5120 M = 256, 136 groups, 242 against 263). Packed IQ3_XXS,
-// whose small GEMM (the generic one) is slower, from 32 groups at 256 rows and on grids of 128
-// groups from 64 rows (17408 x 5120 M = 64 / 128 / 255: 92 / 93 / 135 against 97 / 166 / 309;
-// 6144 x 5120 M = 256, 48 groups: 96 against 114; 5120 x 17408 M = 128, 40 groups: 275 against
-// 148).
+bool small_fp16_shape(int op, int64_t type, int64_t k, int64_t n);
+
+// Whether a product op runs the prefill GEMM (gemm_prefill.hip): a tile of 128 weight rows decoded
+// once per step for up to 256 columns, work split evenly over the CUs, against the small GEMMs'
+// 16-row tiles that decode the weights again for every 4 column tiles. Measured (us per op, graph
+// replays, prefill / the plan it replaces):
+//   34816 x 5120, M = 65 / 256 / 512: IQ3_S 83 / 145 / 257 against 149 / 234 / 353, IQ4_XS 98 / 175 /
+//   317 against 251 / 393 / 607, Q6_K 94 / 151 / 270 against 322 / 249 / 376, IQ2_S 85 / 134 / 254
+//   against 310 / 640 / 1264; 5120 x 6144, M = 65: IQ3_S 31 against 45, Q6_K 32 against 68.
+// On small weights its fixed cost (the table, the K split's parts) shows: 1024 x 5120 M = 100 / 256 /
+// 512 IQ3_S 22 / 24 / 28 against 19 / 22 / 32, 2048 x 5120 M = 100 / 160 23 / 24 against 19 / 29. So from
+// 65 rows on weights of 16M values or more (64 where the fp16 small GEMM's activation layout, the
+// same, served 64), from 129 from 8M values, else from 257. Q2_K, whose other GEMM is the per-slice one,
+// always (12288 x 5120 M = 24 37 against 71; 1024 x 5120 M = 16 21 against 28), up to the K of which one
+// column tile's copy fits the static scratch.
 bool prefill_route(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
-  if (!op_gemm(op) || n < 64) return false;
-  const int64_t groups = (row + 127) / 128 * ((n + 255) / 256);
-  if (xxs_packed(op, type)) return (n >= kPrefillFrom && groups >= 32) || groups >= 128;
-  if (n < kPrefillFrom) return false;
-  return groups >= (type == gguf::kIQ4_XS ? 128 : 64);
+  if (!op_gemm(op) || !gguf::prefill_supported((int)type, op_packed(op))) return false;
+  if (type == gguf::kQ2_K) return gguf::xh_bytes(16, k, (int)type) <= kScratchBytes;  // K <= 209k
+  const int64_t values = row * k;
+  const int64_t from = values >= (16 << 20) ? (small_fp16_shape(op, type, k, 64) ? 64 : 65) : values >= (8 << 20) ? 129 : 257;
+  return n >= from;
+}
+
+// Q6_K products with the sub-scale folded into the fp16 operand, rounded beyond 2048 (xh_decode.h): from
+// 256 rows on grids of 64 tiles of 128 x 256 or more. Elsewhere its operands are exact, as the int8
+// GEMM's are: two MFMAs per slice instead of one.
+bool q6k_rounded(int64_t type, int64_t row, int64_t n) {
+  return type == gguf::kQ6_K && n >= 256 && (row + 127) / 128 * ((n + 255) / 256) >= 64;
+}
+
+// Where the prefill GEMM is the faster one below those rows, but its activation copy is twice the
+// int8 layouts': taken when the library sizes the workspace itself (gguf_mul_mat_alloc), so that the
+// size that gguf_op_workspace_bytes reports stays the smaller one. From 33 rows on weights of 24M
+// values or more (M = 48: Q6_K 5120 x 6144 25 against 33 us, 34816 x 5120 76 against 135; Q4_K 73
+// against 111; IQ2_S 17408 x 5120 41 against 53), packed IQ3_S there from 80M values (34816 x 5120 64
+// against 80, 5120 x 17408 45 against 49; 8192 x 5120 25 against 24) and everything from 49 rows (M =
+// 56: IQ3_S 8192 x 5120 25 against 37); not where the fp16 range plan applies (17408 x 5120 M = 48
+// IQ3_S 42 against 41, Q4_K 45 against 40).
+bool prefill_preferred(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
+  if (prefill_route(op, type, row, k, n)) return true;
+  if (!op_gemm(op) || !gguf::prefill_supported((int)type, op_packed(op))) return false;
+  if (small_fp16_shape(op, type, k, n) && gguf::small_h_range((int)type, row, n)) return false;
+  const int64_t values = row * k;
+  return (n >= 33 && values >= (type == gguf::kIQ3_S ? (80 << 20) : (24 << 20))) || (n >= 49 && values >= (24 << 20));
 }
 
 int64_t vec_mma_from(int op, int64_t type) {
@@ -332,15 +356,15 @@ bool rows_fused(int op, int64_t type, int64_t row, int64_t k, int64_t n, bool ha
   return bb > 0 && gguf::gemv_rows_x_supported((int)type, row, k / 256 * bb, k, n);
 }
 
-// The MFMA products with K <= 8192 run the fp16 small GEMM (X in the xh layout) for packed IQ3_S
-// and Q4_K from 64 to 255 activation rows, and below 64 rows where its one-workgroup-per-CU range
-// plan applies (4..5 row tiles per CU; 33..48 rows for IQ3_S, 17..48 for Q4_K); the rest below the
-// prefill rows the int8 small GEMM (xq layout). Measured at the 27B-layer shapes: from 64 rows the fp16 GEMM's
-// shared decode beats re-decoding the weights per group of 4 column tiles (17408 x 5120 IQ3_S,
-// 128 rows: 84 against 134 us); over K = 17408 (68 blocks in one workgroup's loop, 320
-// workgroups) the int8 GEMM's K split across waves is faster.
+// The MFMA products with K <= 8192 below the prefill GEMM's rows run the fp16 small GEMM (X in the xh
+// layout) for packed IQ3_S and Q4_K from 64 activation rows, and below 64 where its
+// one-workgroup-per-CU range plan applies (4..5 row tiles per CU; 33..48 rows for IQ3_S, 17..48 for
+// Q4_K); the rest the int8 small GEMM (xq layout).
+bool small_fp16_shape(int op, int64_t type, int64_t k, int64_t n) {
+  return op_gemm(op) && k <= 8192 && n >= 17 && gguf::small_h_supported((int)type, op_packed(op));
+}
 bool small_fp16(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
-  if (!op_gemm(op) || k > 8192 || !gguf::small_h_supported((int)type, op_packed(op))) return false;
+  if (!small_fp16_shape(op, type, k, n)) return false;
   return (n >= 64 && !prefill_route(op, type, row, k, n)) || gguf::small_h_range((int)type, row, n);
 }
 
@@ -372,6 +396,15 @@ SplitPlan split_plan(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
   return p;
 }
 
+// Bytes of a prefill product's workspace with its split plan: the xh copy of X, the partial sums and
+// the tile counters. gguf_op_workspace_bytes reports the copy alone: with no more than that the
+// product runs unsplit.
+size_t prefill_split_ws(int64_t type, int64_t row, int64_t k, int64_t n) {
+  const size_t slots = gguf::prefill_slot_bytes(row, k, n);
+  const size_t xh = align256(gguf::xh_bytes(n, k, (int)type));
+  return slots ? xh + slots + align256((size_t)gguf::prefill_counters(row, k, n) * 4) : xh;
+}
+
 // Bytes after the xq copy of X that a split GEMM needs (slots, then its counters).
 size_t split_ws(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
   const SplitPlan p = split_plan(op, type, row, k, n);
@@ -382,16 +415,14 @@ size_t split_ws(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
 
 size_t gguf_op_workspace_bytes(int op, int64_t type, int64_t row, int64_t k, int64_t n, int has_x_q8) {
   if (n <= 0) return 0;
+  if (prefill_route(op, type, row, k, n)) return align256(gguf::xh_bytes(n, k, (int)type));
   if (generic(type)) {
-    if (xxs_packed(op, type) && prefill_route(op, type, row, k, n)) return align256(gguf::xh_bytes(n, k));
     if (op_gemm(op)) return align256(generic_xq(type) ? gguf::xq_bytes(n, k) : gguf_q8_1_bytes(n, k, 1));
     return has_x_q8 || generic_fused(op, type, row, k, n) ? 0 : align256(gguf_q8_1_bytes(n, k, 0));
   }
   if (op_gemm(op)) {
     const bool mmq_layout = !op_packed(op) && type == gguf::kIQ3_S;
-    if (!mmq_layout && ((prefill_route(op, type, row, k, n) && gguf::prefill_uses_xh((int)type, op_packed(op))) ||
-                        small_fp16(op, type, row, k, n)))
-      return align256(gguf::xh_bytes(n, k));
+    if (!mmq_layout && small_fp16(op, type, row, k, n)) return align256(gguf::xh_bytes(n, k, (int)type));
     return align256(mmq_layout ? gguf_q8_1_bytes(n, k, 1) : gguf::xq_bytes(n, k)) + split_ws(op, type, row, k, n);
   }
   if (decode_mma(op, type, row, k, n))  // x_q8 is converted into it
@@ -405,9 +436,12 @@ size_t gguf_op_workspace_bytes(int op, int64_t type, int64_t row, int64_t k, int
 namespace {
 
 // One product whose guards have passed (check_op returned k): the buffer checks, the plan and the
-// launches. Every entry point runs the guards once and then this.
+// launches. Every entry point runs the guards once and then this. prefill: the prefill GEMM runs it
+// (prefill_route or prefill_preferred); its tiles' K is split where the workspace has room for the
+// parts.
 int run_checked(int op, const gguf_view* W, const gguf_view* X, int64_t type, int64_t row, const gguf_view* x_q8,
-                int64_t k, void* y, size_t y_bytes, void* workspace, size_t workspace_bytes, void* stream) {
+                int64_t k, void* y, size_t y_bytes, void* workspace, size_t workspace_bytes, void* stream,
+                bool prefill) {
   const char* name = op_name(op);
   const int64_t n = X->size[0];
   if (n == 0) return GGUF_OK;
@@ -418,7 +452,8 @@ int run_checked(int op, const gguf_view* W, const gguf_view* X, int64_t type, in
   const DeviceScope scope(X->device);
   if (scope.err != hipSuccess) return hip_fail(scope.err, name, "device select");
   // sized on X's device, as the dispatch below decides (some plans depend on its CU count)
-  const size_t need = gguf_op_workspace_bytes(op, type, row, k, n, x_q8 != nullptr);
+  const size_t need = prefill ? align256(gguf::xh_bytes(n, k, (int)type))
+                              : gguf_op_workspace_bytes(op, type, row, k, n, x_q8 != nullptr);
   if (workspace_bytes < need || (need > 0 && !workspace))
     return fail("%s: workspace of %zu bytes needed, got %zu", name, need, workspace_bytes);
   if (reinterpret_cast<uintptr_t>(workspace) % 16 != 0) return fail("%s: workspace must be 16-byte aligned", name);
@@ -428,16 +463,25 @@ int run_checked(int op, const gguf_view* W, const gguf_view* X, int64_t type, in
   const int64_t row_bytes = W->size[1];
   const int ydt = X->dtype;
 
+  if (prefill) {
+    uint8_t* ws = (uint8_t*)workspace;
+    float* part = nullptr;
+    uint32_t* cnt = nullptr;
+    const size_t slots = gguf::prefill_slot_bytes(row, k, n);
+    if (slots && workspace_bytes >= prefill_split_ws(type, row, k, n)) {
+      part = (float*)(ws + align256(gguf::xh_bytes(n, k, (int)type)));
+      cnt = (uint32_t*)((uint8_t*)part + slots);
+    }
+    e = gguf::launch_quantize_xh(X->data, X->dtype, n, k, s01, (int)type, ws, s, cnt,
+                                 cnt ? gguf::prefill_counters(row, k, n) : 0);
+    if (e != hipSuccess) return hip_fail(e, name, "quantize");
+    e = gguf::launch_gemm_prefill((int)type, !q6k_rounded(type, row, n), w, row_bytes, (int)row, (int)k, ws, (int)n, y, ydt, part, cnt, s);
+    if (e != hipSuccess) return hip_fail(e, name, "gemm");
+    return GGUF_OK;
+  }
+
   if (generic(type)) {
     const bool xxs = xxs_packed(op, type);
-    if (xxs && prefill_route(op, type, row, k, n)) {  // IQ3_XXS unit layout: the fp16 prefill GEMM (xh layout)
-      e = gguf::launch_quantize_xh(X->data, X->dtype, n, k, s01, (int)type, workspace, s);
-      if (e != hipSuccess) return hip_fail(e, name, "quantize");
-      e = gguf::launch_gemm_prefill((int)type, true, w, row_bytes, (int)row, (int)k, (const uint8_t*)workspace, (int)n,
-                                    y, ydt, s);
-      if (e != hipSuccess) return hip_fail(e, name, "gemm");
-      return GGUF_OK;
-    }
     if (gemm && generic_xq(type)) {  // the product ops' MMQ arithmetic in the xq layout
       e = gguf::launch_quantize_xq(X->data, X->dtype, n, k, s01, (int)type, false, workspace, s);
       if (e != hipSuccess) return hip_fail(e, name, "quantize");
@@ -497,9 +541,7 @@ int run_checked(int op, const gguf_view* W, const gguf_view* X, int64_t type, in
   // (from vec_mma_from rows on, see decode_mma) with the decode ops' q8_1 arithmetic or the
   // caller's x_q8
   if ((gemm && (packed || type != gguf::kIQ3_S)) || (!gemm && decode_mma(op, type, row, k, n))) {
-    const bool prefill = prefill_route(op, type, row, k, n);
     const bool fp16 = small_fp16(op, type, row, k, n);
-    const bool xh = fp16 || (prefill && gguf::prefill_uses_xh((int)type, packed));
     // a K-split GEMM's slots and counters follow the xq copy; the quantise launch clears the
     // counters
     uint8_t* sws = nullptr;
@@ -513,15 +555,12 @@ int run_checked(int op, const gguf_view* W, const gguf_view* X, int64_t type, in
     }
     if (!gemm && x_q8)
       e = gguf::launch_q8_1_to_xq(x_q8->data, n, k, (int)type, workspace, s, counters, nctr);
-    else if (xh)
+    else if (fp16)
       e = gguf::launch_quantize_xh(X->data, X->dtype, n, k, s01, (int)type, workspace, s);
     else
       e = gguf::launch_quantize_xq(X->data, X->dtype, n, k, s01, (int)type, !gemm, workspace, s, counters, nctr);
     if (e != hipSuccess) return hip_fail(e, name, "quantize");
-    if (prefill)
-      e = gguf::launch_gemm_prefill((int)type, packed, w, row_bytes, (int)row, (int)k, (const uint8_t*)workspace,
-                                    (int)n, y, ydt, s);
-    else if (fp16)
+    if (fp16)
       e = gguf::launch_gemm_small_h((int)type, packed, w, row_bytes, (int)row, (int)k, (const uint8_t*)workspace,
                                     (int)n, y, ydt, s);
     else if (packed)
@@ -572,7 +611,8 @@ int gguf_mul_mat(int op, const gguf_view* W, const gguf_view* X, int64_t type, i
   g_err.clear();
   const int64_t k = check_op(op, W, X, type, row, x_q8);
   if (k < 0) return GGUF_EINVAL;
-  return run_checked(op, W, X, type, row, x_q8, k, y, y_bytes, workspace, workspace_bytes, stream);
+  return run_checked(op, W, X, type, row, x_q8, k, y, y_bytes, workspace, workspace_bytes, stream,
+                     prefill_route(op, type, row, k, X->size[0]));
 }
 
 int gguf_mul_mat_alloc(int op, const gguf_view* W, const gguf_view* X, int64_t type, int64_t row,
@@ -589,13 +629,15 @@ int gguf_mul_mat_alloc(int op, const gguf_view* W, const gguf_view* X, int64_t t
   if (n == 0) return GGUF_OK;
   const DeviceScope scope(X->device);
   if (scope.err != hipSuccess) return hip_fail(scope.err, name, "device select");
-  const size_t need = gguf_op_workspace_bytes(op, type, row, k, n, x_q8 != nullptr);
+  const bool prefill = prefill_preferred(op, type, row, k, n);
+  const size_t need = prefill ? prefill_split_ws(type, row, k, n)
+                              : gguf_op_workspace_bytes(op, type, row, k, n, x_q8 != nullptr);
   void* ws = nullptr;
   if (need) {
     ws = alloc(alloc_ctx, GGUF_ALLOC_WORKSPACE, need);
     if (!ws) return fail("%s: the allocator returned no workspace", name);
   }
-  return run_checked(op, W, X, type, row, x_q8, k, y, y_bytes, ws, need, stream);
+  return run_checked(op, W, X, type, row, x_q8, k, y, y_bytes, ws, need, stream, prefill);
 }
 
 }  // extern "C"
@@ -606,8 +648,20 @@ namespace {
 // the process ends. Host code never uses the array's name as an address (on the host it is only
 // a stand-in for the symbol); each device's address comes from hipGetSymbolAddress with that
 // device current, once, and is kept here.
-constexpr size_t kScratchBytes = GGUF_SCRATCH_BYTES;
 __device__ __align__(256) uint8_t scratch[kScratchBytes];
+
+// Products of the prefill GEMM that this entry point takes although its fp16 activation copy exceeds
+// the scratch: those whose int8 copy (xq, 4.5 KB per 16 rows and K block; block_q8_1_mmq for Q2_K)
+// fits it, on weights and types that the fp16 layout's int8 predecessor served.
+bool noalloc_in_parts(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
+  if (type == gguf::kQ2_K) return align256(gguf_q8_1_bytes(n, k, 1)) <= kScratchBytes;
+  const int64_t groups = (row + 127) / 128 * ((n + 255) / 256);
+  const bool fp16 = xxs_packed(op, type) ? (n >= 256 && groups >= 32) || groups >= 128
+                    : (type == gguf::kIQ3_S || type == gguf::kQ4_K || type == gguf::kQ6_K)
+                        ? (n >= 256 && groups >= 64) || (n < 256 && small_fp16_shape(op, type, k, n))
+                        : false;
+  return !fp16 && align256(gguf::xq_bytes(n, k)) + split_ws(op, type, row, k, n) <= kScratchBytes;
+}
 
 void* g_scratch_ptr[gguf::kMaxDevices] = {};
 std::mutex g_scratch_mu;
@@ -646,13 +700,28 @@ int gguf_mul_mat_noalloc(int op, const gguf_view* W, const gguf_view* X, int64_t
   const DeviceScope scope(X->device);
   if (scope.err != hipSuccess) return hip_fail(scope.err, name, "device select");
   const size_t need = gguf_op_workspace_bytes(op, type, row, k, n, x_q8 != nullptr);
-  if (need > kScratchBytes)
+  const bool prefill = prefill_route(op, type, row, k, n);
+  if (need > kScratchBytes && !(prefill && noalloc_in_parts(op, type, row, k, n)))
     return fail("%s: needs a %zu-byte workspace, more than the %zu-byte static scratch of the no-allocation "
                 "entry point (use gguf_mul_mat with a workspace)", name, need, kScratchBytes);
+  if (y_bytes < (size_t)(n * row * elem_size(X->dtype))) return fail("%s: output buffer too small", name);
   void* ws = nullptr;
   const hipError_t e = scratch_address(X->device, &ws);
   if (e != hipSuccess) return hip_fail(e, name, "scratch address");
-  return run_checked(op, W, X, type, row, x_q8, k, y, y_bytes, ws, kScratchBytes, stream);
+  if (need <= kScratchBytes) return run_checked(op, W, X, type, row, x_q8, k, y, y_bytes, ws, need, stream, prefill);
+  // activation rows in parts whose copy fits the scratch, one after the other on the stream
+  const int64_t es = elem_size(X->dtype);
+  int64_t part = (int64_t)(kScratchBytes / gguf::xh_bytes(16, k, (int)type)) * 16;
+  if (part >= 256) part -= part % 256;  // whole column groups
+  for (int64_t c = 0; c < n; c += part) {
+    gguf_view xp = *X;
+    xp.data = (const uint8_t*)X->data + c * X->stride[0] * es;
+    xp.size[0] = n - c < part ? n - c : part;
+    const int rc = run_checked(op, W, &xp, type, row, x_q8, k, (uint8_t*)y + c * row * es, y_bytes - c * row * es, ws,
+                               kScratchBytes, stream, true);
+    if (rc != GGUF_OK) return rc;
+  }
+  return GGUF_OK;
 }
 
 #define GGUF_OP_Q8(fn, OP)                                                                                    \

@@ -1,27 +1,46 @@
-// Prefill GEMM (many activation rows) on int8 MFMA: Y[c, r] = sum_k X[c, k] * W[r, k].
+// Prefill GEMM (many activation rows) on fp16 MFMA: Y[c, r] = sum_k X[c, k] * W[r, k].
 //
 // Replaces the reference's large-M products (the IQ3 tiled kernel's wide plans,
-// lcpp_owned_iq3_mma.cu:1022-1055, and vendored MMQ, mmq.cuh / mmq-load-tiles.cuh:711,946) with a
-// gfx950 design whose point is operand reuse:
-//  * a workgroup of 4 waves owns a 128-row x 128-column output tile (8 x 8 MFMA tiles of 16 x 16);
-//    wave (wr, wc) accumulates row tiles 4wr..4wr+3 x column tiles 4wc..4wc+3, so every A and B
-//    operand it reads from LDS feeds four MFMAs;
-//  * per 256-value K block the workgroup stages, in LDS,
-//      - A: the block of its 128 weight rows decoded to int8, in MFMA operand order (row tile,
-//        slice, row, 8-byte quarter slot swizzled by row so both the decoders' stores and the
-//        operand reads are free of bank conflicts); each wave decodes two 16-row tiles;
-//      - the per-(row, slice) sub-scales and per-row block scales the epilogue needs;
-//      - B: the xq units (xq.h) of its 8 column tiles, copied by LDS DMA;
-//  * one v_mfma_i32_16x16x32_i8 per (row tile, column tile, slice) is the reference's integer
-//    slice dot; the per-slice epilogue and the block scale are those of the small GEMMs
-//    (Q6_K: two MFMAs per slice, one per 16-value sub-scale; Q4_K: the min term);
-//  * IQ3_S decodes through the 2 KB unsigned grid with the signs applied by VALU (the 32 KB
-//    signed table would leave room for one workgroup per CU).
-// Single-buffered: two workgroups per CU overlap one's staging with the other's MFMAs.
+// lcpp_owned_iq3_mma.cu:1022-1055, and vendored MMQ, mmq.cuh / mmq-load-tiles.cuh) for every type
+// with a product op but IQ1_M (and IQ3 on GGUF rows).
+//
+// Arithmetic. The operand of a weight is its value times its sub-scale, an exact fp16 integer
+// (pf_decode.h), the operand of an activation its q8 value (the xh layout, xq.h). One
+// v_mfma_f32_16x16x32_f16 with a zero accumulator returns sub-scale x integer slice dot, exactly
+// (every partial sum is an integer below 2^24), and the per-slice epilogue is one FMA by the
+// activation scale (IQ4_XS: a multiply by the sub-scale first). The row's block scale d is not
+// applied per slice: each row's accumulator is held in units of the d of the block being summed (e,
+// the last nonzero d; a block with d = 0 decodes to zeros), and is multiplied by e_prev / e_cur when
+// a new block starts and by the last e at the end. The min term of Q4_K, sum over slices of (-dmin / e)
+// m_g s_g, is an integer-weighted sum of the activation sums s_g: one bf16 MFMA per block over m_g
+// (exact in bf16) and s_g in bf16 pieces that add up to it exactly, then one FMA per output by -dmin /
+// e. Q2_K's, over 16-value groups with the fp16 of dmin m_g, is two per half block (two pieces of it).
+//
+// Workgroup: 8 waves over 128 weight rows x 256 / RS activation rows. Wave w owns 2 column tiles of
+// 16 and 8 / RS of the 8 row tiles (RS row parts share a column pair). Its B operands come straight
+// from global memory into registers one step (half a K block) ahead; the decoded weights are shared
+// through LDS, double-buffered, with one LDS-only barrier per step.
+//
+// What bounds it: MFMA and VALU work of a SIMD do not overlap here (a 16 x 16 x 32 MFMA takes 16.4
+// cycles alone, 25 with the 4 FMAs of its epilogue, 35 with 8, at any number of waves, grouped or
+// interleaved), so a step's time is their sum plus what is waited for. The decode of the next step
+// is therefore cut into four parts that run between the MFMA groups of the four slices (table reads
+// of a part at the start of its slice, its operands stored at the end), so that its LDS latencies
+// and the raw loads (a step ahead, two register sets) hide under the MFMAs, and IQ3's two table
+// reads per 8 values are 4 bytes each (a signed table biased by 128; the fp16 grid and sign masks it
+// replaced took four times the LDS bytes).
+//
+// Work split: persistent workgroups (one per CU) over equal contiguous runs of (tile, K block)
+// units, so a grid of 272 tiles takes 272 / 256 rounds, not 2. A run that ends inside a tile leaves
+// its sums in its own slot of the workspace and counts itself in; the workgroup whose count
+// completes the tile adds all parts in K order and writes the output, so the result does not depend
+// on which one that is, and nothing waits.
+#include <algorithm>
 #include <type_traits>
 
 #include "decode.h"
 #include "iq3_tile.h"
+#include "pf_decode.h"
 #include "xh_decode.h"
 #include "xq.h"
 
@@ -29,551 +48,485 @@ namespace gguf {
 
 namespace {
 
-typedef int v4i __attribute__((ext_vector_type(4)));
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 
-constexpr int kPfRowTiles = 8;                  // 128 weight rows per workgroup
-constexpr int kPfColTiles = 8;                  // 128 activation rows per workgroup
-constexpr int kPfSlice = 528;                   // A bytes per (row tile, slice): 16 rows x 32 B + pad
-constexpr int kPfATile = 8 * kPfSlice;          // A bytes per row tile (one block)
-constexpr int kPfA = kPfRowTiles * kPfATile;    // 33,792
-constexpr int kPfB = kPfColTiles * kXqUnit;     // 32,768
-constexpr int kPfBS = kPfColTiles * kXqScaleUnit;  // 4,096
-constexpr int kPfS = kPfRowTiles * 8 * 32;      // sub-scales: [tile][slice][s1 x16 | s2 x16] bytes
-constexpr int kPfD = kPfRowTiles * 16 * 2 * 4;  // [tile][row][d, dmin] fp32
+constexpr int kPfRowTiles = 8;  // 128 weight rows per workgroup
+constexpr int kPfWaves = 8;
+constexpr int kPfThreads = 64 * kPfWaves;
 
-__device__ const Iq3sGrid kIq3sGridPf = kIq3sGrid;
+// The split of a launch: `units` runs of `ub` K blocks over the grid's workgroups; workgroup w takes
+// units [w per + min(w, rem), ...), per or per + 1 of them.
+struct PfPlan {
+  int64_t per, rem;
+  int ub;         // K blocks per unit: 1, or nb where there is no room for partial sums
+  int nrg;        // row groups; tile t = column group t / nrg, row group t % nrg
+};
 
-// A slot of (row tile t, slice u, row j, quarter q): byte offset in the A area. The quarter's
-// slot is q ^ (j >> 2) (as the small GEMM's transposition buffer).
-__device__ __forceinline__ int a_off(int t, int u, int j, int q) {
-  return t * kPfATile + u * kPfSlice + j * 32 + ((q ^ (j >> 2)) & 3) * 8;
+__device__ __forceinline__ int64_t pf_begin(const PfPlan& p, int64_t w) { return w * p.per + min(w, p.rem); }
+// the workgroup that unit x belongs to
+__device__ __forceinline__ int64_t pf_owner(const PfPlan& p, int64_t x) {
+  const int64_t big = p.rem * (p.per + 1);
+  return x < big ? x / (p.per + 1) : p.rem + (x - big) / p.per;
 }
 
-// ------------------------------------------------------------------------- A staging, IQ3_S
-// The lane (decode view L = 8p + s) decodes slice s of rows 2p, 2p+1 of one tile-block and stores
-// the 8 quarters of each row; ex = sign nibble | qh << 4 of each 4-value group.
-__device__ __forceinline__ uint32_t grid_signed(const uint32_t* grid, uint32_t qs, uint32_t ex) {
-  return (uint32_t)apply_signs(grid[qs | ((ex >> 4) << 8)], ex & 0xF);
+// Barrier that orders LDS only: __syncthreads()'s fences also order global memory, for which the
+// compiler may wait for loads still in flight. The scheduling barriers keep each step's code in it.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  __builtin_amdgcn_sched_barrier(0);
 }
 
-__device__ __forceinline__ void stage_iq3_tile(const uint8_t* tile, int64_t row_bytes, int nb, int b,
-                                               const uint32_t* grid, uint8_t* A, uint8_t* S, float* D, int t, int lane) {
-  const int p = lane >> 3, s = lane & 7;
-  const Iq3Fields f = iq3_block_fields(nb, b), l = iq3_lane_fields(p & 1, s);
-  const uint8_t* u = tile + (int64_t)(p >> 1) * kUnitRows * row_bytes;  // rows 2p, 2p+1: unit p >> 1
-  const u32x4 qs = *(const u32x4*)(u + f.qs + l.qs);
-  const uint2 e8 = *(const uint2*)(u + f.e8 + l.e8);
-  const uint32_t l2 = *(const uint16_t*)(u + f.l2 + l.l2);
+// four consecutive rows of one column; vec: their bytes are aligned as a whole
+__device__ __forceinline__ void store_y4(void* y, int64_t i, f4 v, int y_dtype, bool vec, int rows) {
+  if (vec) {
+    if (y_dtype == kF32) {
+      *(f4*)((float*)y + i) = v;
+    } else if (y_dtype == kF16) {
+      uint32_t h[4];
 #pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    uint32_t lo, hi;
-    iq3_tile_ex(r == 0 ? e8.x : e8.y, l2, r, lo, hi);
-    const uint32_t q0 = r == 0 ? qs[0] : qs[2], q1 = r == 0 ? qs[1] : qs[3];
-    uint32_t w[8];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      w[g] = grid_signed(grid, (q0 >> (8 * g)) & 0xFF, (lo >> (8 * g)) & 0xFF);
-      w[4 + g] = grid_signed(grid, (q1 >> (8 * g)) & 0xFF, (hi >> (8 * g)) & 0xFF);
-    }
-    const int j = 2 * p + r;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) *(uint2*)(A + a_off(t, s, j, q)) = make_uint2(w[2 * q], w[2 * q + 1]);
-    // sub-scale ls = 1 + 2 * nibble of (row j, slice s); SC byte 2 (s/2) + r of the row pair, nibble s & 1
-    const uint32_t scb = u[f.sc + l.sc + 2 * (s >> 1) + r];
-    S[(t * 8 + s) * 32 + j] = (uint8_t)(1 + 2 * ((scb >> (4 * (s & 1))) & 0xF));
-    if (s == 0) D[(t * 16 + j) * 2] = half_bits_to_float(*(const uint16_t*)(u + f.d + l.d + 2 * r));
-  }
-}
-
-// ------------------------------------------------------------------------- A staging, raw rows
-// The lane (j = lane & 15, q = lane >> 4) decodes values 8q..8q+7 of every slice of row j of a
-// 16-row tile (blk: row j's block), as the small raw GEMM's A operands.
-template <int TYPE>
-__device__ __forceinline__ void stage_raw_tile(const uint8_t* blk, bool valid, uint8_t* A, uint8_t* S, float* D,
-                                               int t, int lane) {
-  const int j = lane & 15, q = lane >> 4;
-  uint32_t w0[8], w1[8];
-  int s1[8], s2[8];
-  float d = 0.0f, dmin = 0.0f;
-  if (valid) {
-    if constexpr (TYPE == kQ4_K) {
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const uint2 v = *(const uint2*)(blk + 16 + 32 * c + 8 * q);
-        w0[2 * c] = v.x & 0x0F0F0F0Fu;
-        w1[2 * c] = v.y & 0x0F0F0F0Fu;
-        w0[2 * c + 1] = (v.x >> 4) & 0x0F0F0F0Fu;
-        w1[2 * c + 1] = (v.y >> 4) & 0x0F0F0F0Fu;
-      }
-      const uint32_t dm = *(const uint32_t*)blk;
-      d = half_bits_to_float(dm & 0xFFFF);
-      dmin = half_bits_to_float(dm >> 16);
-#pragma unroll
-      for (int u = 0; u < 8; ++u) q4k_scale_min(blk, u, s1[u], s2[u]);
-    } else if constexpr (TYPE == kIQ4_XS) {
-      const int sh = 4 * (q >> 1);
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const uint2 v = *(const uint2*)(blk + 8 + 16 * u + 8 * (q & 1));
-        w0[u] = (uint32_t)iq4nl(v.x, sh);
-        w1[u] = (uint32_t)iq4nl(v.y, sh);
-        s1[u] = iq4xs_ls(blk, u);
-        s2[u] = 0;
-      }
-      d = half_bits_to_float(ld16(blk));
+      for (int e = 0; e < 4; ++e) h[e] = __half_as_ushort(__float2half_rn(v[e]));
+      *(uint2*)((uint16_t*)y + i) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
     } else {
+      uint32_t h[4];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int n = u >> 2, sub = u & 3;
-        const uint64_t l = ld64(blk + 64 * n + 32 * (sub & 1) + 8 * q);
-        const uint64_t h = ld64(blk + 128 + 32 * n + 8 * q);
-        const int lsh = 4 * (sub >> 1), hsh = 2 * sub;
-        w0[u] = (uint32_t)sub32_bytes((((uint32_t)l >> lsh) & 0x0F0F0F0Fu) | ((((uint32_t)h >> hsh) & 0x03030303u) << 4));
-        w1[u] = (uint32_t)sub32_bytes((((uint32_t)(l >> 32) >> lsh) & 0x0F0F0F0Fu) |
-                                      ((((uint32_t)(h >> 32) >> hsh) & 0x03030303u) << 4));
-        s1[u] = (int)(int8_t)blk[192 + 2 * u];
-        s2[u] = (int)(int8_t)blk[193 + 2 * u];
-      }
-      d = half_bits_to_float(ld16(blk + 208));
+      for (int e = 0; e < 4; ++e) h[e] = f32_to_bf16_bits(v[e]);
+      *(uint2*)((uint16_t*)y + i) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
     }
   } else {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) w0[u] = w1[u] = 0, s1[u] = s2[u] = 0;
-  }
-#pragma unroll
-  for (int u = 0; u < 8; ++u) *(uint2*)(A + a_off(t, u, j, q)) = make_uint2(w0[u], w1[u]);
-  if (q == 0) {
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      S[(t * 8 + u) * 32 + j] = (uint8_t)s1[u];
-      S[(t * 8 + u) * 32 + 16 + j] = (uint8_t)s2[u];
-    }
-    D[(t * 16 + j) * 2] = d;
-    D[(t * 16 + j) * 2 + 1] = dmin;
+    for (int e = 0; e < 4; ++e)
+      if (e < rows) store_y(y, i + e, v[e], y_dtype);
   }
 }
 
-// ------------------------------------------------------------------------- the kernel
-// W: weight rows (IQ3_S: the tile layout); xq: X in the xq layout (nct column tiles).
-template <int TYPE, bool TILE>
-__global__ void __launch_bounds__(256, 2) gemm_prefill_kernel(const uint8_t* __restrict__ W, int64_t row_bytes,
-                                                              int nrows, int k, const uint8_t* __restrict__ xq,
-                                                              int nct, int n, void* __restrict__ y, int y_dtype) {
-  __shared__ __attribute__((aligned(16))) uint8_t A[kPfA];
-  __shared__ __attribute__((aligned(16))) uint8_t B[kPfB + kPfBS];
-  __shared__ __attribute__((aligned(16))) uint8_t S[kPfS];
-  __shared__ __attribute__((aligned(16))) float D[kPfD / 4];
-  __shared__ uint32_t grid[TILE ? 512 : 1];
-  constexpr int BS = block_bytes(TYPE);
+template <int TYPE, int RS>
+__global__ void __launch_bounds__(kPfThreads) gemm_prefill_h_kernel(const uint8_t* __restrict__ W, int64_t row_bytes,
+                                                                    int nrows, int k, const uint8_t* __restrict__ xh,
+                                                                    int nct, int n, void* __restrict__ y, int y_dtype,
+                                                                    PfPlan plan, float* __restrict__ part,
+                                                                    uint32_t* __restrict__ cnt) {
+  using Dec = PfDec<TYPE>;
+  using Raw = typename Dec::Raw;
+  constexpr bool IQ3 = pf_iq3(TYPE);   // the unit layouts: a 16-row tile is 4 units
+  constexpr bool MIN = pf_min(TYPE);   // the min term
+  constexpr int AMH = TYPE == kQ2_K ? 2048 : 1024;  // min operands of a half
+  constexpr bool SUB = TYPE == kIQ4_XS;  // sub-scales applied to the dots
+  constexpr bool LO = TYPE == kQ6_KX;   // two planes of operands, added in the MFMA
+  constexpr int RT = kPfRowTiles / RS;  // row tiles per wave
+  constexpr int CG = kPfWaves / RS;     // column pairs per workgroup
+  // row tiles per MFMA group: 4 MFMAs and their 16 FMAs in a row beat 2 and 8 by 3 %; with sub-scales
+  // or two planes two row tiles' operands spill
+  constexpr int GR = SUB || LO ? 1 : 2;
+  constexpr int NG = RT / GR;           // groups per slice
+  constexpr int AD = GR == 1 ? 2 : 1;   // groups ahead that A operands are read
+  constexpr int BD = RS == 1 ? 1 : 2;   // steps ahead that B operands are loaded
+  constexpr int SU = xh_scale_unit(TYPE);
+  constexpr int TB = pf_table_bytes(TYPE);
+  constexpr int kPfA = (LO ? 2 : 1) * kPfPlane;  // operands of a step
+  __shared__ __attribute__((aligned(16))) uint8_t A[2 * kPfA];
+  __shared__ __attribute__((aligned(16))) float RTs[128];
+  __shared__ __attribute__((aligned(16))) float EFs[128];
+  __shared__ __attribute__((aligned(16))) float RMs[MIN ? 256 : 4];
+  __shared__ __attribute__((aligned(16))) uint16_t AMs[MIN ? 2 * AMH : 8];
+  __shared__ __attribute__((aligned(16))) float LSs[SUB ? 2 * 512 : 4];
+  __shared__ __attribute__((aligned(16))) uint4 tbl[TB ? TB / 16 : 1];
+  __shared__ uint32_t last_flag;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wr = wave >> 1, wc = wave & 1;
   const int j = lane & 15, q = lane >> 4;
+  int dj, dq;  // decode lane: row of the tile, index
+  pf_lane(IQ3, lane, dj, dq);
   const int ntiles = (nrows + 15) / 16;
-  const int tile0 = blockIdx.x * kPfRowTiles;
-  const int ct0 = blockIdx.y * kPfColTiles;
   const int nb = k / kQK;
-  const int sbase = (int)xq_scale_base(nct, nb);
-  if constexpr (TILE) {
-    for (int i = threadIdx.x; i < 512; i += 256) grid[i] = kIq3sGridPf.v[i];
-    __syncthreads();  // every wave's decoder reads the whole grid
+  const int cw = wave % CG, r0 = wave / CG * RT;  // column pair and first row tile of this wave
+  // 4 rows of a column in one store
+  const bool vec = nrows % 4 == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;
+
+  if constexpr (TB > 0) {
+    const uint4* src = pf_table<TYPE>();
+    for (int i = threadIdx.x; i < TB / 16; i += kPfThreads) tbl[i] = src[i];
   }
+  const PfLds L0 = {A, RTs, EFs, AMs, RMs, LSs, (const uint8_t*)tbl};
+  const PfLds L1 = {A + kPfA, RTs, EFs, AMs + (MIN ? AMH : 0), RMs + (MIN ? 128 : 0), LSs + (SUB ? 512 : 0),
+                    (const uint8_t*)tbl};
 
-  float acc[4][4][4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r)
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) acc[r][t][v] = 0.0f;
+  // consecutive workgroups go round the 8 XCDs: give each XCD a contiguous range of units, so that
+  // its workgroups share a column group (X stays in its L2)
+  const int64_t nwg = gridDim.x;
+  const int64_t wg = (nwg & 7) == 0 ? (int64_t)(blockIdx.x & 7) * (nwg >> 3) + (blockIdx.x >> 3) : (int64_t)blockIdx.x;
+  int64_t at = pf_begin(plan, wg) * plan.ub;
+  const int64_t end = pf_begin(plan, wg + 1) * plan.ub;
 
-  for (int b = 0; b < nb; ++b) {
-    // ---- stage: B by LDS DMA (16 B per lane per instruction; column tiles past nct re-read the
-    // last one, never stored), A and the scales by the waves' decoders
-#pragma unroll
-    for (int i = 0; i < kPfColTiles / 4; ++i) {
-      const int tt = wave * (kPfColTiles / 4) + i;  // this wave copies column tiles 2w, 2w+1
-      const int ct = ct0 + tt < nct ? ct0 + tt : nct - 1;
-      const uint8_t* src = xq + ((int64_t)ct * nb + b) * kXqUnit;
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-        __builtin_amdgcn_global_load_lds((const void*)(src + c * 1024 + 16 * lane),
-                                         (__attribute__((address_space(3))) void*)(B + tt * kXqUnit + c * 1024), 16,
-                                         0, 0);
-      // scales: 512 B = 32 lanes x 16 B
-      const uint8_t* ssrc = xq + sbase + ((int64_t)ct * nb + b) * kXqScaleUnit;
-      if (lane < 32)
-        __builtin_amdgcn_global_load_lds((const void*)(ssrc + 16 * lane),
-                                         (__attribute__((address_space(3))) void*)(B + kPfB + tt * kXqScaleUnit), 16,
-                                         0, 0);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int t = wave * 2 + i;
-      const int gt = tile0 + t < ntiles ? tile0 + t : ntiles - 1;
-      if constexpr (TILE) {
-        stage_iq3_tile(W + (int64_t)gt * kTileRows * row_bytes, row_bytes, nb, b, grid, A, S, D, t, lane);
-      } else {
-        const int row = gt * 16 + j;
-        const bool valid = row < nrows;
-        stage_raw_tile<TYPE>(W + (int64_t)(valid ? row : 0) * row_bytes + (int64_t)b * BS, valid, A, S, D, t, lane);
-      }
-    }
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
+  while (at < end) {
+    const int64_t tile = at / nb;
+    const int b0 = (int)(at - tile * nb);
+    const int b1 = (int)min((int64_t)nb, (int64_t)b0 + (end - at));
+    at += b1 - b0;
+    const int cgp = (int)(tile / plan.nrg), rg = (int)(tile % plan.nrg);
+    const int tile0 = rg * kPfRowTiles;
 
-    // ---- compute: wave (wr, wc) over its 4 x 4 MFMA tiles; the row's block scale d (and Q4_K's
-    // dmin) is folded into each slice's factor so that one set of accumulators is live
-    float dr[4][4], dmr[4][4];
+    // this wave's column tiles (past nct: the last one again, never stored)
+    const uint8_t* xv[2];
+    const uint8_t* xs[2];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int t = 4 * wr + r;
-      const float4 dd0 = *(const float4*)(D + (t * 16 + 4 * q) * 2);      // d, dmin of rows 4q, 4q+1
-      const float4 dd1 = *(const float4*)(D + (t * 16 + 4 * q + 2) * 2);  // rows 4q+2, 4q+3
-      dr[r][0] = dd0.x; dr[r][1] = dd0.z; dr[r][2] = dd1.x; dr[r][3] = dd1.z;
-      dmr[r][0] = dd0.y; dmr[r][1] = dd0.w; dmr[r][2] = dd1.y; dmr[r][3] = dd1.w;
+    for (int c = 0; c < 2; ++c) {
+      const int ct = min((cgp * CG + cw) * 2 + c, nct - 1);
+      xv[c] = xh + (int64_t)ct * nb * kXhUnit + 16 * lane;
+      xs[c] = xh + xh_scale_base(nct, nb) + (int64_t)ct * nb * SU;
     }
-    const v4i zero = {0, 0, 0, 0};
+    u32x4 bqs[BD][2][4];
+    float dx[2][4];
+    f4 dxn[2];
+    u32x4 mb[2];  // the min term's activation sums of the coming step
+    auto load_bq = [&](u32x4 (&bq)[2][4], int c, int u, int b, int h) {
+      bq[c][u] = *(const u32x4*)(xv[c] + (int64_t)b * kXhUnit + 4096 * h + 1024 * u);
+    };
+    auto load_scales = [&](int b, int h) {
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      long a[4], bo[4];
-      uint32_t s1w[4], s2w[4];
-      uint32_t cw[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int t = 4 * wr + r;
-        a[r] = *(const long*)(A + a_off(t, u, j, q));
-        s1w[r] = *(const uint32_t*)(S + (t * 8 + u) * 32 + 4 * q);
-        if constexpr (TYPE == kQ4_K || TYPE == kQ6_K) s2w[r] = *(const uint32_t*)(S + (t * 8 + u) * 32 + 16 + 4 * q);
+      for (int c = 0; c < 2; ++c) {
+        const uint8_t* s = xs[c] + (int64_t)b * SU;
+        dxn[c] = *(const f4*)(s + 32 * j + 16 * h);
+        if constexpr (TYPE == kQ4_K)
+          if (h == 0) mb[c] = *(const u32x4*)(s + 512 + 32 * j + 16 * (q & 1));
+        if constexpr (TYPE == kQ2_K) mb[c] = *(const u32x4*)(s + 512 + 768 * h + 48 * j + 16 * (q < 3 ? q : 2));
       }
+    };
+    auto take_scales = [&]() {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const int tt = 4 * wc + c;
-        bo[c] = *(const long*)(B + tt * kXqUnit + 64 * lane + 8 * u);
-        cw[c] = *(const uint32_t*)(B + kPfB + tt * kXqScaleUnit + 32 * j + 4 * u);
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) dx[c][u] = dxn[c][u];
+    };
+    // the row tile this wave decodes (tiles past the weight's end, rows past nrows: copies of the
+    // last, never stored)
+    const uint8_t* wp;
+    if constexpr (IQ3) wp = W + (int64_t)min(tile0 + wave, ntiles - 1) * kTileRows * row_bytes;
+    else wp = W + (int64_t)min((tile0 + wave) * 16 + dj, nrows - 1) * row_bytes;
+
+    float e = 1.0f;
+    Raw raw0, raw1;
+    f4 acc[RT][2];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) acc[r][0] = acc[r][1] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+
+    // One step: the 4 slices of half H of the block in A[H], with the decode of the following half
+    // (raw bytes `raw`) into the other buffer; bnx: the block whose half 1 - H is the next step; bld:
+    // the next block; braw: the block whose half 1 - H is decoded two steps on
+    auto step = [&](auto HC, int bnx, Raw& raw, int bld, int braw) {
+      constexpr int H = decltype(HC)::value;
+      constexpr int HN = 1 - H;
+      const uint8_t* Ab = A + H * kPfA;
+      const PfLds& LN = H == 0 ? L1 : L0;
+      typename Dec::Ctx ctx;
+      typename Dec::Tmp tmp[2];
+      u32x4 mbc[2];
+      if constexpr (MIN) {  // before load_scales overwrites them
+        mbc[0] = mb[0];
+        mbc[1] = mb[1];
       }
+      // the LDS reads that the step starts with go out first: what follows covers their latency
+      h8 a[AD + 1][GR];  // the A operands (and sub-scales) of groups g .. g + AD
+      h8 al[AD + 1][GR];
+      f4 ls[AD + 1][GR];
+      f4 p[GR][2];
+      auto read_a = [&](int g) {
+        const int u = g / NG, r = g % NG * GR;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        int s1[4], s2[4];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          if constexpr (TYPE == kIQ3_S || TYPE == kQ4_K) s1[v] = (int)((s1w[r] >> (8 * v)) & 0xFF);
-          else s1[v] = (int)(int8_t)((s1w[r] >> (8 * v)) & 0xFF);
-          if constexpr (TYPE == kQ4_K) s2[v] = (int)((s2w[r] >> (8 * v)) & 0xFF);
-          if constexpr (TYPE == kQ6_K) s2[v] = (int)(int8_t)((s2w[r] >> (8 * v)) & 0xFF);
+        for (int i = 0; i < GR; ++i) {
+          a[g % (AD + 1)][i] = *(const h8*)(Ab + pf_off(r0 + r + i, u, j, q));
+          if constexpr (LO) al[g % (AD + 1)][i] = *(const h8*)(Ab + kPfPlane + pf_off(r0 + r + i, u, j, q));
+          if constexpr (SUB)
+            ls[g % (AD + 1)][i] = *(const f4*)((H == 0 ? L0.LS : L1.LS) + ((r0 + r + i) * 4 + u) * 16 + 4 * q);
         }
+      };
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const float cd = TYPE == kQ4_K ? half_bits_to_float(cw[c] & 0xFFFF) : __uint_as_float(cw[c]);
-          if constexpr (TYPE == kQ6_K) {
-            const v4i c0 = __builtin_amdgcn_mfma_i32_16x16x32_i8(q < 2 ? a[r] : 0, bo[c], zero, 0, 0, 0);
-            const v4i c1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(q < 2 ? 0 : a[r], bo[c], zero, 0, 0, 0);
+      for (int g = 0; g < AD; ++g) read_a(g);
+      load_scales(bnx, HN);
+      u32x4 (&bq)[2][4] = bqs[BD == 1 ? 0 : H];
+      __builtin_amdgcn_sched_barrier(0);
+      Dec::begin(raw, ctx, HN, e, LN, wave, dj, dq);
+      Dec::template issue<0>(ctx, tmp[0], LN);
+      if (H == 0 || TYPE == kQ2_K) {  // a new block: rescale every row to its e; the min term
 #pragma unroll
-            for (int v = 0; v < 4; ++v)
-              acc[r][c][v] = fmaf((float)(__mul24(c0[v], s1[v]) + __mul24(c1[v], s2[v])), cd * dr[r][v], acc[r][c][v]);
-          } else {
-            const v4i cc = __builtin_amdgcn_mfma_i32_16x16x32_i8(a[r], bo[c], zero, 0, 0, 0);
+        for (int r = 0; r < RT; ++r) {
+          f4 rt;
+          if constexpr (H == 0) rt = *(const f4*)(RTs + (r0 + r) * 16 + 4 * q);
+          if constexpr (MIN) {
+            const uint16_t* am = (H == 0 ? L0.AM : L1.AM) + ((r0 + r) * 16 + j) * 8;
+            const f4 rm = *(const f4*)((H == 0 ? L0.RM : L1.RM) + (r0 + r) * 16 + 4 * q);
+            const b8 am8 = __builtin_bit_cast(b8, *(const u32x4*)am);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) acc[r][c][v] = fmaf((float)__mul24(cc[v], s1[v]), cd * dr[r][v], acc[r][c][v]);
-            if constexpr (TYPE == kQ4_K) {
-              const float cs = cd * (float)(int)(int16_t)(cw[c] >> 16);
+            for (int c = 0; c < 2; ++c) {
+              const u32x4 bz = q < (TYPE == kQ4_K ? 2 : 3) ? mbc[c] : u32x4{0, 0, 0, 0};
+              f4 pm = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am8, __builtin_bit_cast(b8, bz), zero, 0, 0, 0);
+              if constexpr (TYPE == kQ2_K)
+                pm = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, *(const u32x4*)(am + 1024)),
+                                                             __builtin_bit_cast(b8, bz), pm, 0, 0, 0);
 #pragma unroll
-              for (int v = 0; v < 4; ++v) acc[r][c][v] = fmaf(-(float)s2[v] * dmr[r][v], cs, acc[r][c][v]);
+              for (int v = 0; v < 4; ++v) {
+                if constexpr (H == 0) acc[r][c][v] *= rt[v];
+                acc[r][c][v] = fmaf(pm[v], rm[v], acc[r][c][v]);
+              }
             }
+          } else {
+            acc[r][0] *= rt;
+            acc[r][1] *= rt;
           }
         }
       }
       __builtin_amdgcn_sched_barrier(0);
-    }
-    __syncthreads();  // the next block's staging overwrites A, B, S, D
-  }
+      // group g = (slice, GR row tiles): the A operands AD groups on are read, 2 GR MFMAs issued, and
+      // the previous group's results folded into acc
+      auto fold = [&](int g, const f4 (&lg)[GR]) {
+        const int u = g / NG, r = g % NG * GR;
+#pragma unroll
+        for (int i = 0; i < GR; ++i)
+#pragma unroll
+          for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+              const float x = SUB ? p[i][c][v] * lg[i][v] : p[i][c][v];
+              acc[r + i][c][v] = fmaf(x, dx[c][u], acc[r + i][c][v]);
+            }
+      };
+#define GGUF_PF_SLICE(U)                                                                                              \
+  if constexpr (U < 3) Dec::template issue<(U < 3 ? U + 1 : 3)>(ctx, tmp[(U + 1) & 1], LN);                           \
+  _Pragma("unroll") for (int gr = 0; gr < NG; ++gr) {                                                                 \
+    const int g = U * NG + gr;                                                                                        \
+    f4 nx[GR][2], lg[GR];                                                                                             \
+    if constexpr (SUB) _Pragma("unroll") for (int i = 0; i < GR; ++i) lg[i] = ls[(g + AD) % (AD + 1)][i];             \
+    if (GR > 1 && g + AD < 4 * NG) read_a(g + AD);                                                                    \
+    _Pragma("unroll") for (int i = 0; i < GR; ++i) _Pragma("unroll") for (int c = 0; c < 2; ++c) nx[i][c] =           \
+        __builtin_amdgcn_mfma_f32_16x16x32_f16(a[g % (AD + 1)][i], __builtin_bit_cast(h8, bq[c][U]), zero, 0, 0, 0);  \
+    if constexpr (LO) _Pragma("unroll") for (int i = 0; i < GR; ++i) _Pragma("unroll") for (int c = 0; c < 2; ++c)    \
+        nx[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[g % (AD + 1)][i], __builtin_bit_cast(h8, bq[c][U]),      \
+                                                          nx[i][c], 0, 0, 0);                                         \
+    if (g > 0) fold(g - 1, lg);                                                                                       \
+    if (GR == 1 && g + AD < 4 * NG) read_a(g + AD);                                                                   \
+    _Pragma("unroll") for (int i = 0; i < GR; ++i) _Pragma("unroll") for (int c = 0; c < 2; ++c) p[i][c] = nx[i][c];  \
+    __builtin_amdgcn_sched_barrier(0);                                                                                \
+  }                                                                                                                   \
+  load_bq(bq, 0, U, BD == 1 ? bnx : bld, BD == 1 ? HN : H);                                                           \
+  load_bq(bq, 1, U, BD == 1 ? bnx : bld, BD == 1 ? HN : H);                                                           \
+  Dec::template finish<U>(ctx, tmp[U & 1], LN, wave, dj, dq);                                                         \
+  __builtin_amdgcn_sched_barrier(0);
+      GGUF_PF_SLICE(0)
+      GGUF_PF_SLICE(1)
+      GGUF_PF_SLICE(2)
+      GGUF_PF_SLICE(3)
+#undef GGUF_PF_SLICE
+      // last, so that no wait for B operands or scales waits for it: loads return in order
+      Dec::load(raw, wp, row_bytes, nb, braw, HN, dj, dq);
+      fold(4 * NG - 1, ls[(4 * NG - 1) % (AD + 1)]);
+      take_scales();
+    };
 
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int t = tile0 + 4 * wr + r;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int col = (ct0 + 4 * wc + c) * kXqCols + j;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int row = t * 16 + 4 * q + v;
-        if (col < n && t < ntiles && row < nrows) store_y(y, (int64_t)col * nrows + row, acc[r][c][v], y_dtype);
-      }
-    }
-  }
-}
-
-// ------------------------------------------------------------------------- fp16-operand variant
-// IQ3_S and Q4_K: the weight value times its slice sub-scale is an integer of at most 465 (IQ3_S)
-// or 945 (Q4_K), exact in fp16, and so are the activation's q8 values (the xh layout). One
-// v_mfma_f32_16x16x32_f16 with a zero accumulator then returns sub-scale x integer slice dot
-// exactly (every partial sum is an integer below 2^24), already in fp32, and the per-slice
-// epilogue is one FMA by the activation scale. Q6_K: the 16-value sub-scale goes into the decoded
-// operand, (q - 32) * sc, so a 32-value slice with two sub-scales is one MFMA as well (the int8
-// GEMM needs one per sub-scale); that product is exact up to 2048 in magnitude and rounds to
-// fp16 beyond (xh_decode.h). The row's block scale d is not applied per
-// slice: each row's accumulator is held in units of the d of the block being summed (e, the last
-// nonzero d; a block with d = 0 decodes to zeros), and is multiplied by e_prev / e_cur when a new
-// block starts and by the last e at the end. The Q4_K min term, sum over slices of
-// (-dmin * m / e) x (the fp16 sum of the slice's x, the MMQ form), is a K = 4 fp32 product per
-// half block: one v_mfma_f32_16x16x4f32 into the accumulator.
-//
-// Workgroup: NW waves over 128 weight rows x 32 NW activation rows. Wave w owns column tiles 2w,
-// 2w+1 against all 8 row tiles (16 accumulator tiles); its B operands (4 KB per column tile and
-// half block) come straight from global memory into registers one step ahead, so only the
-// decoded weights are shared through LDS, double-buffered, with one barrier per step (half
-// block). Each wave decodes 8 / NW row tiles per step from raw bytes it loaded two steps ahead.
-constexpr int kHA = kPfRowTiles * 4 * kHRegion;    // 33,280 per buffer (half a K block)
-
-template <int TYPE, int NW>
-__global__ void __launch_bounds__(64 * NW, 8 / NW) gemm_prefill_h_kernel(const uint8_t* __restrict__ W,
-                                                                         int64_t row_bytes, int nrows, int k,
-                                                                         const uint8_t* __restrict__ xh, int nct,
-                                                                         int n, void* __restrict__ y, int y_dtype) {
-  constexpr bool XXS = TYPE == kIQ3_XXS;
-  constexpr bool IQ3 = TYPE == kIQ3_S || XXS;  // the unit layouts: a 16-row tile is 4 units
-  constexpr bool MIN = TYPE == kQ4_K;  // the min term
-  constexpr int TPW = 8 / NW;  // row tiles a wave decodes per step
-  using Raw = typename std::conditional<
-      XXS, RawXxsH,
-      typename std::conditional<IQ3, RawIq3, typename std::conditional<MIN, RawQ4k, RawQ6k>::type>::type>::type;
-  __shared__ __attribute__((aligned(16))) uint8_t A[2 * kHA];
-  __shared__ __attribute__((aligned(16))) float RT[128];
-  __shared__ __attribute__((aligned(16))) float EF[128];
-  __shared__ __attribute__((aligned(16))) float AM[MIN ? 2 * 512 : 4];
-  __shared__ __attribute__((aligned(16))) uint32_t GH[IQ3 ? 1024 : 4];
-  __shared__ __attribute__((aligned(16))) uint2 SM[16];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int j = lane & 15, q = lane >> 4;
-  const int ntiles = (nrows + 15) / 16;
-  const int tile0 = blockIdx.x * kPfRowTiles;
-  const int nb = k / kQK;
-  if constexpr (IQ3) {
-    iq3_half_tables_to_lds(GH, SM, threadIdx.x, 64 * NW, XXS);
-  }
-
-  // this wave's column tiles (past nct: the last one again, never stored)
-  const uint8_t* xv[2];
-  const uint8_t* xs[2];
-#pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    const int ct = min((int)blockIdx.y * 2 * NW + 2 * wave + c, nct - 1);
-    xv[c] = xh + (int64_t)ct * nb * kXhUnit + 16 * lane;
-    xs[c] = xh + xh_scale_base(nct, nb) + (int64_t)ct * nb * kXhScaleUnit + 32 * j;
-  }
-  // B operands of the current step: slice u of column tile c, refilled with the next step's as
-  // soon as the slice's MFMAs are issued; its scales (and Q4_K's sums) in a second set
-  u32x4 bq[2][4];
-  float dx[2][4], dxn[2][4], sq[2], sqn[2];
-  auto load_bq = [&](int c, int u, int b, int h) {
-    bq[c][u] = *(const u32x4*)(xv[c] + (int64_t)b * kXhUnit + 4096 * h + 1024 * u);
-  };
-  auto load_scales = [&](int b, int h) {
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const f4 v = *(const f4*)(xs[c] + (int64_t)b * kXhScaleUnit + 16 * h);
-      dxn[c][0] = v[0];
-      dxn[c][1] = v[1];
-      dxn[c][2] = v[2];
-      dxn[c][3] = v[3];
-      if constexpr (MIN) sqn[c] = *(const float*)(xs[c] + (int64_t)b * kXhScaleUnit + 512 + 16 * h + 4 * q);
-    }
-  };
-  auto take_scales = [&]() {
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) dx[c][u] = dxn[c][u];
-      sq[c] = sqn[c];
-    }
-  };
-  // this wave's decode rows (tiles past the weight's end, rows past nrows: copies, never stored)
-  const uint8_t* wp[TPW];
-#pragma unroll
-  for (int i = 0; i < TPW; ++i) {
-    const int t = wave * TPW + i;
-    if constexpr (IQ3) {
-      wp[i] = W + (int64_t)min(tile0 + t, ntiles - 1) * kTileRows * row_bytes;
-    } else {
-      wp[i] = W + (int64_t)min((tile0 + t) * 16 + j, nrows - 1) * row_bytes;
-    }
-  }
-  Raw raw[TPW];
-  float e[TPW];
-  auto load_w = [&](int b, int h) {
-#pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-      if constexpr (IQ3) load_step(raw[i], wp[i], row_bytes, nb, b, h, j, q);
-      else load_step(raw[i], wp[i] + (int64_t)b * block_bytes(TYPE), h, q);
-    }
-  };
-  auto decode = [&](int h) {
-    uint8_t* Ab = A + h * kHA;
-#pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-      const int t = wave * TPW + i;
-      if constexpr (IQ3) decode_step(raw[i], h, GH, SM, Ab, RT, EF, e[i], t, j, q);
-      else if constexpr (MIN) decode_step(raw[i], h, AM + h * 512, Ab, RT, EF, e[i], t, j, q);
-      else decode_step(raw[i], h, Ab, RT, EF, e[i], t, j, q);
-    }
-  };
-
-  f4 acc[8][2];
-#pragma unroll
-  for (int r = 0; r < 8; ++r) acc[r][0] = acc[r][1] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-  const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-  // One step: 4 slices x 8 row tiles x 2 column tiles. Software-pipelined: the next A operand is
-  // read while the current pair of MFMAs runs, and a pair's results are folded into acc one
-  // row tile later. nb_, nh: the step whose B operands refill the registers.
-  auto compute = [&](int h, int bnext, int hnext) {
-    const uint8_t* Ab = A + h * kHA;
-    if (h == 0) {  // a new block: rescale every row to its e
-#pragma unroll
-      for (int r = 0; r < 8; ++r) {
-        const f4 rt = *(const f4*)(RT + r * 16 + 4 * q);
-        acc[r][0] *= rt;
-        acc[r][1] *= rt;
-      }
-    }
-    h8 a = *(const h8*)(Ab + h_off(0, 0, j, q));
-    f4 p0 = zero, p1 = zero;
+    // prologue: the first half decoded, the second's raw bytes and the first's operands in flight
+    Dec::load(raw0, wp, row_bytes, nb, b0, 0, dj, dq);
+    Dec::load(raw1, wp, row_bytes, nb, b0, 1, dj, dq);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
 #pragma unroll
-      for (int r = 0; r < 8; ++r) {
-        const int rn = r == 7 ? 0 : r + 1, un = r == 7 ? u + 1 : u;
-        h8 an = a;
-        if (un < 4) an = *(const h8*)(Ab + h_off(rn, un, j, q));
-        const f4 n0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(h8, bq[0][u]), zero, 0, 0, 0);
-        const f4 n1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(h8, bq[1][u]), zero, 0, 0, 0);
-        if (u > 0 || r > 0) {
-          const int rp = r == 0 ? 7 : r - 1, upv = r == 0 ? u - 1 : u;
+      for (int h = 0; h < BD; ++h) {
+        load_bq(bqs[h], 0, u, b0, h);
+        load_bq(bqs[h], 1, u, b0, h);
+      }
+    }
+    load_scales(b0, 0);
+    __syncthreads();  // the table; the previous tile's readers of A, RT and EF are done
+    {
+      typename Dec::Ctx ctx;
+      typename Dec::Tmp tmp;
+      Dec::begin(raw0, ctx, 0, e, L0, wave, dj, dq);
+      Dec::template issue<0>(ctx, tmp, L0);
+      Dec::template finish<0>(ctx, tmp, L0, wave, dj, dq);
+      Dec::template issue<1>(ctx, tmp, L0);
+      Dec::template finish<1>(ctx, tmp, L0, wave, dj, dq);
+      Dec::template issue<2>(ctx, tmp, L0);
+      Dec::template finish<2>(ctx, tmp, L0, wave, dj, dq);
+      Dec::template issue<3>(ctx, tmp, L0);
+      Dec::template finish<3>(ctx, tmp, L0, wave, dj, dq);
+    }
+    take_scales();
+    Dec::load(raw0, wp, row_bytes, nb, min(b0 + 1, b1 - 1), 0, dj, dq);
+    lds_barrier();
+    for (int b = b0; b < b1; ++b) {
+      const int bn = min(b + 1, b1 - 1);  // past the end: the last block again (never used; its
+                                          // decode leaves e and EF as they are)
+      step(std::integral_constant<int, 0>{}, b, raw1, bn, bn);
+      lds_barrier();
+      step(std::integral_constant<int, 1>{}, bn, raw0, bn, min(b + 2, b1 - 1));
+      lds_barrier();
+    }
 #pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            acc[rp][0][v] = fmaf(p0[v], dx[0][upv], acc[rp][0][v]);
-            acc[rp][1][v] = fmaf(p1[v], dx[1][upv], acc[rp][1][v]);
+    for (int r = 0; r < RT; ++r) {
+      const f4 ef = *(const f4*)(EFs + (r0 + r) * 16 + 4 * q);
+      acc[r][0] *= ef;
+      acc[r][1] *= ef;
+    }
+
+    if (b1 - b0 < nb) {  // a part of the tile's K
+      constexpr int kSlot = RT * 2 * kPfThreads * 4;  // floats
+      const int64_t first = pf_owner(plan, tile * nb);
+      const int parts = (int)(pf_owner(plan, tile * nb + nb - 1) - first) + 1;
+      const int mine = (int)(wg - first);
+      // slot of a workgroup's part: 2 w where the part continues a tile, 2 w + 1 where it starts one
+      auto slot_of = [&](int i) { return part + ((first + i) * 2 + (i == 0 ? 1 : 0)) * kSlot; };
+      uint64_t* out = (uint64_t*)slot_of(mine);
+#pragma unroll
+      for (int i = 0; i < RT * 2; ++i) {
+        const f4 v = acc[i >> 1][i & 1];
+        const uint64_t lo = (uint64_t)__float_as_uint(v[0]) | ((uint64_t)__float_as_uint(v[1]) << 32);
+        const uint64_t hi = (uint64_t)__float_as_uint(v[2]) | ((uint64_t)__float_as_uint(v[3]) << 32);
+        __hip_atomic_store(out + (2 * i) * kPfThreads + threadIdx.x, lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(out + (2 * i + 1) * kPfThreads + threadIdx.x, hi, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+      }
+      // every wave's stores are complete before the workgroup counts itself in
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (threadIdx.x == 0)
+        last_flag = __hip_atomic_fetch_add(cnt + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __syncthreads();
+      if (last_flag != (uint32_t)parts - 1) continue;
+      asm volatile("" ::: "memory");
+      // all parts in K order; this workgroup's own come from its registers
+      f4 own[RT * 2];
+#pragma unroll
+      for (int i = 0; i < RT * 2; ++i) own[i] = acc[i >> 1][i & 1];
+      for (int z = 0; z < parts; ++z) {
+        uint64_t* in = (uint64_t*)slot_of(z);
+#pragma unroll
+        for (int i = 0; i < RT * 2; ++i) {
+          f4 v = own[i];
+          if (z != mine) {
+            const uint64_t lo = __hip_atomic_load(in + (2 * i) * kPfThreads + threadIdx.x, __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_AGENT);
+            const uint64_t hi = __hip_atomic_load(in + (2 * i + 1) * kPfThreads + threadIdx.x, __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_AGENT);
+            v = f4{__uint_as_float((uint32_t)lo), __uint_as_float((uint32_t)(lo >> 32)), __uint_as_float((uint32_t)hi),
+                   __uint_as_float((uint32_t)(hi >> 32))};
           }
+          acc[i >> 1][i & 1] = z == 0 ? v : acc[i >> 1][i & 1] + v;
         }
-        p0 = n0;
-        p1 = n1;
-        a = an;
-      }
-      load_bq(0, u, bnext, hnext);  // slice u's operands are consumed: the next step's
-      load_bq(1, u, bnext, hnext);
-    }
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      acc[7][0][v] = fmaf(p0[v], dx[0][3], acc[7][0][v]);
-      acc[7][1][v] = fmaf(p1[v], dx[1][3], acc[7][1][v]);
-    }
-    if constexpr (MIN) {  // the min term of the half block
-#pragma unroll
-      for (int r = 0; r < 8; ++r) {
-        const float am = AM[h * 512 + (r * 4 + q) * 16 + j];
-#pragma unroll
-        for (int c = 0; c < 2; ++c) acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(am, sq[c], acc[r][c], 0, 0, 0);
       }
     }
-  };
 
+    const int col0 = (cgp * CG + cw) * 2 * kXqCols + j;
 #pragma unroll
-  for (int i = 0; i < TPW; ++i) e[i] = 1.0f;
-  load_w(0, 0);
+    for (int r = 0; r < RT; ++r) {
+      const int t = tile0 + r0 + r;
+      const int row = t * 16 + 4 * q;
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    load_bq(0, u, 0, 0);
-    load_bq(1, u, 0, 0);
-  }
-  load_scales(0, 0);
-  if constexpr (IQ3) __syncthreads();  // the decode tables
-  decode(0);
-  load_w(0, 1);
-  take_scales();
-  __syncthreads();
-  for (int b = 0; b < nb; ++b) {
-    const int bn = min(b + 1, nb - 1);  // past the end: block nb - 1 again (never computed)
-    // sched_barrier: the decode's arithmetic on the raw bytes stays after the MFMAs (hoisted
-    // into them it makes the whole step wait for the raw loads of the step after)
-    load_scales(b, 1);
-    compute(0, b, 1);
-    __builtin_amdgcn_sched_barrier(0);
-    decode(1);
-    load_w(bn, 0);
-    take_scales();
-    __syncthreads();
-    load_scales(bn, 0);
-    compute(1, bn, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    decode(0);  // at the last block a repeat of it, which leaves e and EF as they are
-    load_w(bn, 1);
-    take_scales();
-    __syncthreads();
-  }
-
-  const int col0 = ((int)blockIdx.y * 2 * NW + 2 * wave) * kXqCols + j;
-#pragma unroll
-  for (int r = 0; r < 8; ++r) {
-    const int t = tile0 + r;
-    const f4 ef = *(const f4*)(EF + r * 16 + 4 * q);
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const int col = col0 + c * kXqCols;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int row = t * 16 + 4 * q + v;
-        if (col < n && t < ntiles && row < nrows) store_y(y, (int64_t)col * nrows + row, acc[r][c][v] * ef[v], y_dtype);
+      for (int c = 0; c < 2; ++c) {
+        const int col = col0 + c * kXqCols;
+        if (col < n && row < nrows) store_y4(y, (int64_t)col * nrows + row, acc[r][c], y_dtype, vec, nrows - row);
       }
     }
   }
 }
 
-template <int TYPE, int NW>
-void launch_prefill_h_t(const uint8_t* W, int64_t row_bytes, int nrows, int k, const uint8_t* xh, int n, void* y,
-                        int y_dtype, hipStream_t stream) {
-  const int nct = (int)xq_col_tiles(n);
-  const int ntiles = (nrows + 15) / 16;
-  const dim3 grid((unsigned)((ntiles + kPfRowTiles - 1) / kPfRowTiles), (unsigned)((nct + 2 * NW - 1) / (2 * NW)));
-  gemm_prefill_h_kernel<TYPE, NW><<<grid, 64 * NW, 0, stream>>>(W, row_bytes, nrows, k, xh, nct, n, y, y_dtype);
+// The split of one product: row parts (a workgroup's columns are 256 / rs), tiles of 128 rows x those
+// columns, workgroups.
+struct PfShape {
+  int rs;
+  int64_t tiles, wgs;
+};
+
+// At most one workgroup per CU, each of at least 4 K blocks (a part of a tile costs its workgroup
+// about two blocks' time to publish and another to add up). rs: least estimated time, in us
+// fixed(rs) + blocks per workgroup x block(rs), a block's time growing with the workgroups at work.
+// IQ3_S, K = 5120, slopes and intercepts over rows and K splits: block 3.5 / 2.3 / 1.7 us with a few
+// workgroups and 5.6 / 3.0 / 2.3 with 256 for rs = 1 / 2 / 4, fixed 20 / 16 / 14. Measured at rs =
+// 1 / 2 / 4: 1024 rows M = 256 48 / 32 / 25 us, 8192 rows M = 128 49 / 33 / 34, 34816 rows M = 100
+// 133 / 89 / 115, M = 512 271 / 305 / 400.
+PfShape pf_shape(int64_t nrows, int64_t k, int64_t n) {
+  static const double fixed[3] = {20, 16, 14}, few[3] = {3.5, 2.3, 1.7}, full[3] = {5.6, 3.0, 2.3};
+  const int64_t nct = xq_col_tiles(n), nb = k / kQK, nrg = (nrows + 127) / 128, cus = device_cus();
+  PfShape best{1, 0, 0};
+  double least = 0;
+  for (int i = 0; i < 3; ++i) {
+    const int rs = 1 << i;
+    const int64_t per = 16 / rs, tiles = nrg * ((nct + per - 1) / per), units = tiles * nb;
+    const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(cus, units / 4));
+    const double t = fixed[i] + (double)((units + wgs - 1) / wgs) * (few[i] + (full[i] - few[i]) * (double)wgs / (double)cus);
+    if (i == 0 || t < least) least = t, best = {rs, tiles, wgs};
+  }
+  return best;
+}
+
+template <int TYPE, int RS>
+void launch_prefill_h(const PfShape& s, const uint8_t* W, int64_t row_bytes, int nrows, int k, const uint8_t* xh, int n,
+                      void* y, int y_dtype, float* part, uint32_t* cnt, hipStream_t stream) {
+  const int64_t nb = k / kQK, tiles = s.tiles;
+  const bool split = part != nullptr;
+  PfPlan p;
+  p.ub = split ? 1 : (int)nb;
+  p.nrg = (nrows + 127) / 128;
+  const int64_t units = split ? tiles * nb : tiles;
+  const int64_t wgs = split ? s.wgs : std::min<int64_t>(device_cus(), tiles);
+  p.per = units / wgs;
+  p.rem = units % wgs;
+  gemm_prefill_h_kernel<TYPE, RS><<<dim3((unsigned)wgs), kPfThreads, 0, stream>>>(
+      W, row_bytes, nrows, k, xh, (int)xq_col_tiles(n), n, y, y_dtype, p, part, cnt);
 }
 
 template <int TYPE>
-void launch_prefill_h(const uint8_t* W, int64_t row_bytes, int nrows, int k, const uint8_t* xh, int n, void* y,
-                      int y_dtype, hipStream_t stream) {
-  const int64_t groups = (int64_t)((nrows + 127) / 128) * ((xq_col_tiles(n) + 15) / 16);
-  if (groups >= 256) launch_prefill_h_t<TYPE, 8>(W, row_bytes, nrows, k, xh, n, y, y_dtype, stream);
-  else launch_prefill_h_t<TYPE, 4>(W, row_bytes, nrows, k, xh, n, y, y_dtype, stream);
-}
-
-template <int TYPE, bool TILE>
-void launch_prefill_t(const uint8_t* W, int64_t row_bytes, int nrows, int k, const uint8_t* xq, int n, void* y,
-                      int y_dtype, hipStream_t stream) {
-  const int nct = (int)xq_col_tiles(n);
-  const int ntiles = (nrows + 15) / 16;
-  const dim3 grid((unsigned)((ntiles + kPfRowTiles - 1) / kPfRowTiles), (unsigned)((nct + kPfColTiles - 1) / kPfColTiles));
-  gemm_prefill_kernel<TYPE, TILE><<<grid, 256, 0, stream>>>(W, row_bytes, nrows, k, xq, nct, n, y, y_dtype);
+void launch_prefill_t(const uint8_t* W, int64_t row_bytes, int nrows, int k, const uint8_t* xh, int n, void* y,
+                      int y_dtype, float* part, uint32_t* cnt, hipStream_t stream) {
+  const PfShape s = pf_shape(nrows, k, n);
+  switch (s.rs) {
+    case 1: launch_prefill_h<TYPE, 1>(s, W, row_bytes, nrows, k, xh, n, y, y_dtype, part, cnt, stream); break;
+    case 2: launch_prefill_h<TYPE, 2>(s, W, row_bytes, nrows, k, xh, n, y, y_dtype, part, cnt, stream); break;
+    default: launch_prefill_h<TYPE, 4>(s, W, row_bytes, nrows, k, xh, n, y, y_dtype, part, cnt, stream); break;
+  }
 }
 
 }  // namespace
 
-// Whether the prefill GEMM of this type takes X in the xh layout (else xq).
-bool prefill_uses_xh(int type, bool packed) { return packed || type == kQ4_K || type == kQ6_K; }
+// Whether the prefill GEMM serves the type: packed IQ3, and GGUF rows of every other type with a
+// product op but IQ3 and IQ1_M.
+bool prefill_supported(int type, bool packed) {
+  if (packed) return type == kIQ3_S || type == kIQ3_XXS;
+  return type == kQ4_K || type == kQ6_K || type == kIQ4_XS || type == kQ2_K || type == kIQ2_XXS || type == kIQ2_XS ||
+         type == kIQ2_S;
+}
 
-// Large-M products; xq: X in the xq layout, or the xh layout where prefill_uses_xh. packed: IQ3_S
-// or IQ3_XXS in its unit layout (nrows % 16 == 0).
-hipError_t launch_gemm_prefill(int type, bool packed, const uint8_t* W, int64_t row_bytes, int nrows, int k,
-                               const uint8_t* xq, int n, void* y, int y_dtype, hipStream_t stream) {
-  if (packed) {
-    if (type == kIQ3_XXS) launch_prefill_h<kIQ3_XXS>(W, row_bytes, nrows, k, xq, n, y, y_dtype, stream);
-    else launch_prefill_h<kIQ3_S>(W, row_bytes, nrows, k, xq, n, y, y_dtype, stream);
-  } else {
-    switch (type) {
-      case kQ4_K: launch_prefill_h<kQ4_K>(W, row_bytes, nrows, k, xq, n, y, y_dtype, stream); break;
-      case kIQ4_XS: launch_prefill_t<kIQ4_XS, false>(W, row_bytes, nrows, k, xq, n, y, y_dtype, stream); break;
-      case kQ6_K: launch_prefill_h<kQ6_K>(W, row_bytes, nrows, k, xq, n, y, y_dtype, stream); break;
-      default: return hipErrorInvalidValue;
-    }
+// Tile counters of the split plan, and the bytes of its partial sums (two slots per workgroup; 0: the
+// runs are whole tiles and nothing is split).
+int64_t prefill_counters(int64_t nrows, int64_t k, int64_t n) { return pf_shape(nrows, k, n).tiles; }
+size_t prefill_slot_bytes(int64_t nrows, int64_t k, int64_t n) {
+  const int64_t nb = k / kQK;
+  const PfShape s = pf_shape(nrows, k, n);
+  if (s.tiles * nb % s.wgs == 0 && s.tiles * nb / s.wgs % nb == 0) return 0;
+  return (size_t)(s.wgs * 2) * (16 / s.rs) * 2 * 4096;
+}
+
+// Large-M products; xh: X in the xh layout of the type; part: prefill_slot_bytes of workspace, with
+// prefill_counters counters that the quantise launch cleared at cnt, or null: no tile is split. exact: Q6_K's
+// operands without the rounding beyond 2048 (two MFMAs per slice).
+hipError_t launch_gemm_prefill(int type, bool exact, const uint8_t* W, int64_t row_bytes, int nrows, int k, const uint8_t* xh, int n,
+                               void* y, int y_dtype, float* part, uint32_t* cnt, hipStream_t stream) {
+#define GGUF_PF(T) \
+  case T: launch_prefill_t<T>(W, row_bytes, nrows, k, xh, n, y, y_dtype, part, cnt, stream); break;
+  switch (type == kQ6_K && exact ? kQ6_KX : type) {
+    GGUF_PF(kQ6_KX)
+    GGUF_PF(kIQ3_S)
+    GGUF_PF(kIQ3_XXS)
+    GGUF_PF(kQ4_K)
+    GGUF_PF(kQ6_K)
+    GGUF_PF(kIQ4_XS)
+    GGUF_PF(kQ2_K)
+    GGUF_PF(kIQ2_XXS)
+    GGUF_PF(kIQ2_XS)
+    GGUF_PF(kIQ2_S)
+    default: return hipErrorInvalidValue;
   }
+#undef GGUF_PF
   return hipGetLastError();
 }
 

@@ -1,9 +1,10 @@
 // Small-batch GEMM on fp16 MFMA for IQ3_S (tile layout) and Q4_K rows: Y[c, r] = sum_k X[c, k] *
-// W[r, k] for 64..255 activation rows (product ops below the prefill GEMM's rows).
+// W[r, k] for product ops below the prefill GEMM's rows: from 64 activation rows on small weights, and
+// the range plan's 17..48.
 //
 // Replaces the reference's tiled products at these row counts (lcpp_owned_iq3_mma.cu:614-1096 for
 // packed IQ3_S, vendored MMQ for Q4_K) with a gfx950 design on the exact fp16 route of the prefill
-// GEMM (xh_decode.h): a weight value times its slice sub-scale is an exact fp16 integer, so one
+// GEMM (pf_decode.h): a weight value times its slice sub-scale is an exact fp16 integer, so one
 // v_mfma_f32_16x16x32_f16 returns sub-scale x integer slice dot exactly in fp32 and the per-slice
 // epilogue is one FMA by the activation scale (the int8-MFMA route needs an integer multiply, a
 // conversion and an FMA per output element and slice).
@@ -220,7 +221,7 @@ __global__ void __launch_bounds__(64 * (DPT * RT + NM * MW), RANGE ? 1 : 4) gemm
   for (int i = 0; i < TPM; ++i) tix[i] = min(tm + MW * i, RT - 1);
   const int ct = min(ctw, nct - 1);
   const uint8_t* xv = xh + (int64_t)ct * nb * kXhUnit + 16 * lane;
-  const uint8_t* xs = xh + xh_scale_base(nct, nb) + (int64_t)ct * nb * kXhScaleUnit + 32 * j;
+  const uint8_t* xs = xh + xh_scale_base(nct, nb) + (int64_t)ct * nb * xh_scale_unit(TYPE) + 32 * j;
   // two named sets (blocks of even and odd index), each refilled in place with the block two on
   // once consumed: one step of prefetch is shorter than the load latency under this traffic
   struct BSet {
@@ -229,9 +230,12 @@ __global__ void __launch_bounds__(64 * (DPT * RT + NM * MW), RANGE ? 1 : 4) gemm
   };
   auto load_b = [&](BSet& o, int s, int b) {
     o.bq[s] = *(const u32x4*)(xv + (int64_t)b * kXhUnit + 1024 * s);
-    o.dq[s] = *(const float*)(xs + (int64_t)b * kXhScaleUnit + 4 * s);
+    o.dq[s] = *(const float*)(xs + (int64_t)b * xh_scale_unit(TYPE) + 4 * s);
     if constexpr (!IQ3)
-      if ((s & 3) == 0) o.sqv[s >> 2] = *(const float*)(xs + (int64_t)b * kXhScaleUnit + 512 + 4 * (s + q));
+      if ((s & 3) == 0) {  // the two bf16 pieces of slice s + q's sum
+        const uint8_t* p = xs + (int64_t)b * xh_scale_unit(TYPE) + 512 + 2 * (s + q);
+        o.sqv[s >> 2] = __uint_as_float(ld16(p) << 16) + __uint_as_float(ld16(p + 16) << 16);
+      }
   };
   f4 acc[TPM];
 #pragma unroll

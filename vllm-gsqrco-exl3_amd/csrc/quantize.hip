@@ -146,33 +146,6 @@ __device__ __forceinline__ void xq_store(uint8_t* y, int k, int c, int kk, int n
   }
 }
 
-// The prefill GEMM's fp16 layout (xq.h, "xh"); same thread mapping and values as xq_store (MMQ
-// arithmetic: for DS4 the min term's activation side is the fp16 sum of x, widened to fp32).
-template <bool DS4>
-__device__ __forceinline__ void xh_store(uint8_t* y, int k, int c, int kk, int nct, uint32_t lo, uint32_t hi, float d,
-                                         float xsum) {
-  const int nb = k / kQK;
-  const int b = kk / kQK;
-  const int u = (kk / kQ81) & 7, q = (kk / 8) & 3;
-  const int t = c / kXqCols, j = c % kXqCols;
-  const int64_t unit = (int64_t)t * nb + b;
-  uint32_t h[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const uint32_t w = e < 2 ? lo : hi;
-    const int sh = 16 * (e & 1);
-    const float f0 = (float)(int8_t)((w >> sh) & 0xFF), f1 = (float)(int8_t)((w >> (sh + 8)) & 0xFF);
-    h[e] = (uint32_t)__half_as_ushort(__float2half_rn(f0)) | ((uint32_t)__half_as_ushort(__float2half_rn(f1)) << 16);
-  }
-  *(uint4*)(y + unit * kXhUnit + 1024 * u + 16 * (16 * q + j)) = make_uint4(h[0], h[1], h[2], h[3]);
-  if (q == 0) {
-    uint8_t* sc = y + xh_scale_base(nct, nb) + unit * kXhScaleUnit + 32 * j + 4 * u;
-    const float dd = DS4 ? half_bits_to_float(__half_as_ushort(__float2half_rn(d))) : d;
-    *(float*)sc = dd;
-    if constexpr (DS4) *(float*)(sc + 512) = half_bits_to_float(__half_as_ushort(__float2half_rn(xsum)));
-  }
-}
-
 // Workgroup (0, 0) of a quantise launch clears `zero_words` dwords at `zero` (the split GEMM's
 // counters, which the GEMM that follows in stream order reads; null: none).
 __device__ __forceinline__ void clear_words(uint32_t* zero, int zero_words) {
@@ -182,7 +155,7 @@ __device__ __forceinline__ void clear_words(uint32_t* zero, int zero_words) {
 
 // Thread (x, y) of the grid: values 8 x .. 8 x + 7 of activation row c0 + y (rows past n, the last
 // column tile's padding, quantise zeros). k % 32 == 0, so a slice's four threads exit together.
-template <int DT, bool VEC, bool DS4, bool XH = false>
+template <int DT, bool VEC, bool DS4>
 __global__ void __launch_bounds__(256) quantize_xq_kernel(const void* __restrict__ x, uint8_t* __restrict__ y, int k,
                                                           int64_t s01, int n, int nct, int c0, uint32_t* zero,
                                                           int zero_words) {
@@ -233,8 +206,116 @@ __global__ void __launch_bounds__(256) quantize_xq_kernel(const void* __restrict
     b += __shfl_xor(b, 1, 64);
     xsum = a + b;
   }
-  if constexpr (XH) xh_store<DS4>(y, k, c, kk, nct, lo, hi, d, xsum);
-  else xq_store<VEC, DS4>(y, k, c, kk, nct, lo, hi, d, qsum, xsum);
+  xq_store<VEC, DS4>(y, k, c, kk, nct, lo, hi, d, qsum, xsum);
+}
+
+// X -> the xh layout (xq.h), MMQ arithmetic. One workgroup per (K block, column tile): wave w
+// quantises slices 2w, 2w + 1; lane (j = lane & 15, q = lane >> 4) the values 8q .. 8q + 7 of both in
+// activation row 16t + j, so that a wave's stores are two contiguous KB (with consecutive values of
+// one row in consecutive lanes every 16-byte store was a cache line of its own: 2048 x 5120 bf16
+// 24.7 us). VL: 8 values of a row are aligned 16-byte loads.
+template <int DT, int LAYOUT, bool VL>
+__global__ void __launch_bounds__(256) quantize_xh_kernel(const void* __restrict__ x, uint8_t* __restrict__ y, int k,
+                                                          int64_t s01, int n, int nct, int t0, uint32_t* zero,
+                                                          int64_t zero_words) {
+  if (zero != nullptr && blockIdx.x == 0 && blockIdx.y == 0)
+    for (int64_t i = threadIdx.x; i < zero_words; i += 256) zero[i] = 0u;
+  constexpr int SU = LAYOUT == kD2S6 ? 2048 : 1024;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, j = lane & 15, q = lane >> 4;
+  const int nb = k / kQK, b = blockIdx.x, t = t0 + (int)blockIdx.y;
+  const int c = t * kXqCols + j;
+  const int64_t unit = (int64_t)t * nb + b;
+  float v[2][8], am[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int64_t at = (int64_t)c * s01 + b * kQK + 64 * w + 32 * i + 8 * q;
+    if (c < n) {
+      if constexpr (VL && DT == kF32) {
+        const float4 f0 = *(const float4*)((const float*)x + at), f1 = *(const float4*)((const float*)x + at + 4);
+        v[i][0] = f0.x, v[i][1] = f0.y, v[i][2] = f0.z, v[i][3] = f0.w;
+        v[i][4] = f1.x, v[i][5] = f1.y, v[i][6] = f1.z, v[i][7] = f1.w;
+      } else if constexpr (VL) {
+        const u32x4 f = *(const u32x4*)((const uint16_t*)x + at);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const uint32_t hb = (f[e >> 1] >> (16 * (e & 1))) & 0xFFFF;
+          v[i][e] = DT == kF16 ? half_bits_to_float(hb) : __uint_as_float(hb << 16);
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[i][e] = ldx<DT>(x, at + e);
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[i][e] = 0.0f;
+    }
+    float m = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf(v[i][e]));
+    m = fmaxf(m, __shfl_xor(m, 16, 64));
+    am[i] = fmaxf(m, __shfl_xor(m, 32, 64));
+  }
+  if constexpr (LAYOUT == kD2S6) am[0] = am[1] = fmaxf(am[0], am[1]);
+  uint8_t* sc = y + xh_scale_base(nct, nb) + unit * SU;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int u = 2 * w + i;
+    float d = 0.0f;
+    int qv[8];
+    if (am[i] != 0.0f) {
+      const float d_inv = 127.0f / am[i];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) qv[e] = (int)(int8_t)(int)roundf(v[i][e] * d_inv);
+      d = 1.0f / d_inv;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) qv[e] = 0;
+    }
+    uint32_t h[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      h[e] = (uint32_t)__half_as_ushort(__float2half_rn((float)qv[2 * e])) |
+             ((uint32_t)__half_as_ushort(__float2half_rn((float)qv[2 * e + 1])) << 16);
+    *(uint4*)(y + unit * kXhUnit + 1024 * u + 16 * lane) = make_uint4(h[0], h[1], h[2], h[3]);
+    if constexpr (LAYOUT != kD4) d = half_bits_to_float(__half_as_ushort(__float2half_rn(d)));
+    if (q == 0) *(float*)(sc + 32 * j + 4 * u) = d;
+    if constexpr (LAYOUT != kD4) {
+      // the MMQ quantiser's sums in its order: 4-value lane sums ((x0 + x1) + x2) + x3, then the xor
+      // butterfly over the slice's 8 lanes (DS4) or the group's 4 (D2S6), of which this lane holds
+      // two neighbours
+      float a = ((v[i][0] + v[i][1]) + v[i][2]) + v[i][3];
+      float bb = ((v[i][4] + v[i][5]) + v[i][6]) + v[i][7];
+      if constexpr (LAYOUT == kDS4) {
+        a += __shfl_xor(a, 32, 64);
+        bb += __shfl_xor(bb, 32, 64);
+      }
+      a += __shfl_xor(a, 16, 64);
+      bb += __shfl_xor(bb, 16, 64);
+      float s = half_bits_to_float(__half_as_ushort(__float2half_rn(a + bb)));
+      if constexpr (LAYOUT == kD2S6) {
+        int sq = 0;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sq += qv[e];
+        sq += __shfl_xor(sq, 16, 64);
+        if ((u & 3) == 3) s = d * (float)sq;  // groups 6, 7 of each 128 values; exact
+      }
+      // bf16 pieces, exact: 8 + 8 bits hold an fp16, 8 + 8 + 8 an fp32
+      uint32_t piece[3];
+      float r = s;
+#pragma unroll
+      for (int z = 0; z < 3; ++z) {
+        piece[z] = f32_to_bf16_bits(r);
+        r = fabsf(s) < INFINITY ? r - __uint_as_float(piece[z] << 16) : 0.0f;
+      }
+      if constexpr (LAYOUT == kDS4) {
+        if (q < 2) *(uint16_t*)(sc + 512 + 32 * j + 16 * q + 2 * u) = (uint16_t)(q == 0 ? piece[0] : piece[1]);
+      } else if ((q & 1) == 0) {  // group 2 (u & 3) + (q >> 1) of half u >> 2
+        uint8_t* p = sc + 512 + 768 * (u >> 2) + 48 * j + 2 * (2 * (u & 3) + (q >> 1));
+#pragma unroll
+        for (int z = 0; z < 3; ++z) *(uint16_t*)(p + 16 * z) = (uint16_t)piece[z];
+      }
+    }
+  }
 }
 
 // block_q8_1 bytes of X (a caller's x_q8) -> the xq layout with the same values and fp16 scales.
@@ -293,28 +374,39 @@ hipError_t launch_quantize_xq(const void* x, int dtype, int64_t n, int64_t k, in
   return hipGetLastError();
 }
 
-// X [n, k] -> the xh layout at y (xh_bytes(n, k) bytes), MMQ arithmetic, for weights of `type`.
+// X [n, k] -> the xh layout at y (xh_bytes(n, k, type) bytes), MMQ arithmetic, for weights of `type`;
+// the first launch also clears zero_words dwords at zero (null: none).
 hipError_t launch_quantize_xh(const void* x, int dtype, int64_t n, int64_t k, int64_t s01, int type, void* y,
-                              hipStream_t stream) {
+                              hipStream_t stream, uint32_t* zero, int64_t zero_words) {
   if (n == 0) return hipSuccess;
-  const int nct = (int)xq_col_tiles(n), rows = nct * kXqCols;
-  const unsigned gx = (unsigned)((k / 8 + 255) / 256);
-  const bool ds4 = type == kQ4_K;
-  for (int c0 = 0; c0 < rows; c0 += kQuantRowsPerLaunch) {
-    const dim3 grid(gx, (unsigned)std::min(rows - c0, kQuantRowsPerLaunch));
-#define GGUF_QXH(DT)                                                                                               \
-  if (ds4)                                                                                                         \
-    quantize_xq_kernel<DT, false, true, true><<<grid, 256, 0, stream>>>(x, (uint8_t*)y, (int)k, s01, (int)n, nct, c0, \
-                                                                        nullptr, 0);                              \
-  else                                                                                                             \
-    quantize_xq_kernel<DT, false, false, true><<<grid, 256, 0, stream>>>(x, (uint8_t*)y, (int)k, s01, (int)n, nct, c0, \
-                                                                         nullptr, 0);
+  const int nct = (int)xq_col_tiles(n);
+  const int layout = mmq_layout(type);
+  const int64_t es = dtype == kF32 ? 4 : 2;
+  const bool vl = reinterpret_cast<uintptr_t>(x) % 16 == 0 && s01 * es % 16 == 0;
+  for (int t0 = 0; t0 < nct; t0 += kQuantRowsPerLaunch) {
+    const dim3 grid((unsigned)(k / kQK), (unsigned)std::min(nct - t0, kQuantRowsPerLaunch));
+    uint32_t* z = t0 == 0 ? zero : nullptr;
+#define GGUF_QXH3(DT, L, V) \
+  quantize_xh_kernel<DT, L, V><<<grid, 256, 0, stream>>>(x, (uint8_t*)y, (int)k, s01, (int)n, nct, t0, z, zero_words)
+#define GGUF_QXH2(DT, L)          \
+  if (vl) GGUF_QXH3(DT, L, true); \
+  else GGUF_QXH3(DT, L, false);
+#define GGUF_QXH(DT)                               \
+  if (layout == kDS4) {                            \
+    GGUF_QXH2(DT, kDS4)                            \
+  } else if (layout == kD2S6) {                    \
+    GGUF_QXH2(DT, kD2S6)                           \
+  } else {                                         \
+    GGUF_QXH2(DT, kD4)                             \
+  }
     switch (dtype) {
       case kF32: GGUF_QXH(kF32) break;
       case kF16: GGUF_QXH(kF16) break;
       default: GGUF_QXH(kBF16) break;
     }
 #undef GGUF_QXH
+#undef GGUF_QXH2
+#undef GGUF_QXH3
   }
   return hipGetLastError();
 }

@@ -1,14 +1,11 @@
-// fp16 decode of weight blocks for the fp16-operand MFMA GEMMs (the prefill GEMM's fp16 variant
-// and the small GEMM): IQ3_S and IQ3_XXS in their unit layouts (iq3_tile.h), Q4_K and Q6_K rows,
-// decoded to fp16
-// values with the slice (Q6_K: 16-value) sub-scale applied (exact integers: at most 465 for
-// IQ3_S, 945 for Q4_K; Q6_K's up to 4064 round above 2048), in the A-operand order of
-// v_mfma_f32_16x16x32_f16.
+// fp16 decode of weight blocks for the fp16-operand MFMA GEMMs: the raw loads of IQ3_S and IQ3_XXS in
+// their unit layouts (iq3_tile.h) and of Q6_K rows, which the prefill GEMM decodes (pf_decode.h), and
+// the small GEMM's Q4_K decode: fp16 values with the slice sub-scale applied (exact integers, at most
+// 945), in the A-operand order of v_mfma_f32_16x16x32_f16.
 //
-// A decoding lane (row j = lane & 15, part q = lane >> 4) handles one row of a 16-row tile for
-// half a K block (4 slices): IQ3_S slice 4h + q of row j; Q4_K quarter q (8 values) of each of
-// the half block's 4 slices of row j. The decoded half block of row tile t sits at h_off(t, ...)
-// of the caller's A area.
+// A decoding lane (row j, part q) handles one row of a 16-row tile for half a K block (4 slices): IQ3
+// slice 4h + q of row j; Q4_K and Q6_K quarter q (8 values) of each of the half block's 4 slices of row
+// j. The small GEMM's decoded half block of row tile t sits at h_off(t, ...) of the caller's A area.
 //
 // Block scales: each row's accumulator is held in units of e, the last nonzero d of the row's
 // blocks so far (a block with d = 0 decodes to zeros). At a block start the decoder writes the
@@ -28,41 +25,6 @@ typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
 constexpr int kHRegion = 1040;                     // A bytes per (row tile, slice): 16 rows x 64 B + pad
-
-// fp16 bits of a small positive integer
-constexpr uint32_t small_int_half(uint32_t v) {
-  int e = 0;
-  while ((v >> (e + 1)) != 0) ++e;
-  return ((uint32_t)(e + 15) << 10) | ((v - (1u << e)) << (10 - e));
-}
-static_assert(small_int_half(1) == 0x3C00 && small_int_half(15) == 0x4B80, "fp16 bits");
-
-// The IQ3_S grid as fp16: entry i = the 4 grid values of index i, 2 per dword
-struct Iq3sGridHalf {
-  uint32_t v[1024];
-};
-constexpr Iq3sGridHalf make_iq3s_grid_half() {
-  Iq3sGridHalf g{};
-  for (int i = 0; i < 512; ++i) {
-    const uint32_t w = kIq3sGrid.v[i];
-    g.v[2 * i] = small_int_half(w & 0xFF) | (small_int_half((w >> 8) & 0xFF) << 16);
-    g.v[2 * i + 1] = small_int_half((w >> 16) & 0xFF) | (small_int_half(w >> 24) << 16);
-  }
-  return g;
-}
-__device__ const Iq3sGridHalf kIq3sGridHalf = make_iq3s_grid_half();
-
-// The IQ3_XXS grid as fp16 (entries 0..255 in the first 512 dwords)
-constexpr Iq3sGridHalf make_iq3xxs_grid_half() {
-  Iq3sGridHalf g{};
-  for (int i = 0; i < 256; ++i) {
-    const uint32_t w = kIq3xxsGrid.v[i];
-    g.v[2 * i] = small_int_half(w & 0xFF) | (small_int_half((w >> 8) & 0xFF) << 16);
-    g.v[2 * i + 1] = small_int_half((w >> 16) & 0xFF) | (small_int_half(w >> 24) << 16);
-  }
-  return g;
-}
-__device__ const Iq3sGridHalf kIq3xxsGridHalf = make_iq3xxs_grid_half();
 
 // A slot of (row tile t, slice u of the half block, row j, quarter q): the quarter's 16 bytes sit
 // in slot q ^ g(j) of the row, g(j) = ((j >> 1) ^ (j >> 3)) & 3, which keeps the operand reads
@@ -137,62 +99,6 @@ __device__ __forceinline__ float next_scale(float d, float& e, float* RT, float*
   return en;
 }
 
-__device__ __forceinline__ void decode_step(const RawIq3& w, int h, const uint32_t* gh, const uint2* sm, uint8_t* A,
-                                            float* RT, float* EF, float& e, int t, int j, int sp) {
-  const int s = 4 * h + sp;
-  const float d = half_bits_to_float(w.d);
-  if (h == 0) next_scale(d, e, RT, EF, t * 16 + j);
-  uint32_t lo, hi;
-  iq3_tile_ex(w.e8, w.l2, j & 1, lo, hi);
-  const uint32_t nib = (w.sc >> (4 * (s & 1))) & 0xF;
-  const _Float16 ls = d != 0.0f ? (_Float16)(float)(1 + 2 * nib) : (_Float16)0.0f;
-  const h2 lsh = {ls, ls};
-  uint32_t v[16];
-#pragma unroll
-  for (int g = 0; g < 8; ++g) {
-    const uint32_t qb = ((g < 4 ? w.qs.x : w.qs.y) >> (8 * (g & 3))) & 0xFF;
-    const uint32_t ex = ((g < 4 ? lo : hi) >> (8 * (g & 3))) & 0xFF;
-    const uint2 gv = *(const uint2*)(gh + 2 * (qb | ((ex >> 4) << 8)));
-    const uint2 sg = sm[ex & 0xF];
-    v[2 * g] = h2_bits(bits_h2(gv.x ^ sg.x) * lsh);
-    v[2 * g + 1] = h2_bits(bits_h2(gv.y ^ sg.y) * lsh);
-  }
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-    *(uint4*)(A + h_off(t, sp, j, q)) = make_uint4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
-}
-
-// IQ3_XXS: value = d * ls * w / 4 (ls = 2 * scale + 1, w the signed grid byte): the operand is
-// w * ls (at most 62 * 31 = 1922, exact in fp16) and the row's scale d / 4. The second word of
-// each 8-value group takes bits 4..6 of the group's 7-bit sign index and their parity with bits
-// 0..3 (ksigns_iq2xs), all four parities from two three-way xors (bit 7g of t ^ t >> 3 ^ a >> 6,
-// t = a ^ a >> 1 ^ a >> 2, is the xor of bits 7g..7g+6).
-__device__ __forceinline__ void decode_step(const RawXxsH& w, int h, const uint32_t* gh, const uint2* sm, uint8_t* A,
-                                            float* RT, float* EF, float& e, int t, int j, int sp) {
-  const float d = half_bits_to_float(w.d) * 0.25f;
-  if (h == 0) next_scale(d, e, RT, EF, t * 16 + j);
-  const uint32_t a = w.aux;
-  const uint32_t t3 = a ^ (a >> 1) ^ (a >> 2);
-  const uint32_t par = t3 ^ (t3 >> 3) ^ (a >> 6);
-  const uint32_t hi = ((par << 3) & 0x01020408u) | ((a >> 4) & ~0x01020408u);
-  const _Float16 ls = d != 0.0f ? (_Float16)(float)(2 * (a >> 28) + 1) : (_Float16)0.0f;
-  const h2 lsh = {ls, ls};
-  uint32_t v[16];
-#pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    const uint32_t qw = (g < 2 ? w.qs.x : w.qs.y) >> (16 * (g & 1));
-    const uint2 g0 = *(const uint2*)(gh + 2 * (qw & 0xFF)), g1 = *(const uint2*)(gh + 2 * ((qw >> 8) & 0xFF));
-    const uint2 s0 = sm[(a >> (7 * g)) & 0xF], s1 = sm[(hi >> (7 * g)) & 0xF];
-    v[4 * g] = h2_bits(bits_h2(g0.x ^ s0.x) * lsh);
-    v[4 * g + 1] = h2_bits(bits_h2(g0.y ^ s0.y) * lsh);
-    v[4 * g + 2] = h2_bits(bits_h2(g1.x ^ s1.x) * lsh);
-    v[4 * g + 3] = h2_bits(bits_h2(g1.y ^ s1.y) * lsh);
-  }
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-    *(uint4*)(A + h_off(t, sp, j, q)) = make_uint4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
-}
-
 // Q4_K: fp16 (1024 + nibble) by a byte permute, then one packed FMA gives nibble x sc exactly.
 __device__ __forceinline__ void decode_step(const RawQ4k& w, int h, float* AM, uint8_t* A, float* RT, float* EF,
                                             float& e, int t, int j, int q) {
@@ -245,48 +151,6 @@ __device__ __forceinline__ void load_step(RawQ6k& w, const uint8_t* blk, int h, 
   w.qh = ld64(blk + 128 + 32 * h + 8 * q);
   w.sc = ld64(blk + 192 + 8 * h);
   w.d = ld16(blk + 208);
-}
-
-// Q6_K: fp16 (1024 + q) by a byte permute, q - 32 by one packed subtract (exact), then times the
-// 16-value sub-scale by one packed multiply. The product (q - 32) * sc is exact in fp16 up to 2048
-// in magnitude; beyond (sub-scales above 64) an odd product rounds to an even neighbour, 2^-12
-// relative at most. The lane's 8 values of slice 4h + sub share sub-scale 2 sub + (q >> 1).
-__device__ __forceinline__ void decode_step(const RawQ6k& w, int h, uint8_t* A, float* RT, float* EF, float& e,
-                                            int t, int j, int q) {
-  const float d = half_bits_to_float(w.d);
-  if (h == 0) next_scale(d, e, RT, EF, t * 16 + j);
-  else e = d != 0.0f ? d : e;
-  const bool nz = d != 0.0f;
-  const h2 bias = {(_Float16)-1056.0f, (_Float16)-1056.0f};
-#pragma unroll
-  for (int sub = 0; sub < 4; ++sub) {
-    const uint64_t l = (sub & 1) ? w.lb : w.la;
-    const int lsh = 4 * (sub >> 1), hsh = 2 * sub;
-    const uint32_t x0 = (((uint32_t)l >> lsh) & 0x0F0F0F0Fu) | ((((uint32_t)w.qh >> hsh) & 0x03030303u) << 4);
-    const uint32_t x1 = (((uint32_t)(l >> 32) >> lsh) & 0x0F0F0F0Fu) | ((((uint32_t)(w.qh >> 32) >> hsh) & 0x03030303u) << 4);
-    const int scv = (int)(int8_t)((w.sc >> (8 * (2 * sub + (q >> 1)))) & 0xFF);
-    const _Float16 scf = nz ? (_Float16)(float)scv : (_Float16)0.0f;
-    const h2 mul = {scf, scf};
-    const uint32_t w0 = h2_bits((bits_h2(__builtin_amdgcn_perm(0x64646464u, x0, 0x04010400u)) + bias) * mul);
-    const uint32_t w1 = h2_bits((bits_h2(__builtin_amdgcn_perm(0x64646464u, x0, 0x04030402u)) + bias) * mul);
-    const uint32_t w2 = h2_bits((bits_h2(__builtin_amdgcn_perm(0x64646464u, x1, 0x04010400u)) + bias) * mul);
-    const uint32_t w3 = h2_bits((bits_h2(__builtin_amdgcn_perm(0x64646464u, x1, 0x04030402u)) + bias) * mul);
-    *(uint4*)(A + h_off(t, sub, j, q)) = make_uint4(w0, w1, w2, w3);
-  }
-}
-
-// The IQ3_S decode tables in LDS: the fp16 grid (GH, 1024 dwords) and the 16 sign masks (SM),
-// written by threads tid = 0 .. nt - 1 of the workgroup; the caller synchronises.
-__device__ __forceinline__ void iq3_half_tables_to_lds(uint32_t* GH, uint2* SM, int tid, int nt, bool xxs = false) {
-  if (xxs) {
-    for (int i = tid; i < 512; i += nt) GH[i] = kIq3xxsGridHalf.v[i];
-  } else {
-    for (int i = tid; i < 1024; i += nt) GH[i] = kIq3sGridHalf.v[i];
-  }
-  if (tid < 16) {
-    const uint32_t nib = tid;
-    SM[nib] = make_uint2(((nib & 1u) << 15) | ((nib & 2u) << 30), ((nib & 4u) << 13) | ((nib & 8u) << 28));
-  }
 }
 
 }  // namespace

@@ -43,18 +43,25 @@ __host__ __device__ inline size_t xq_bytes(int64_t n, int64_t k) {
 //           bytes at 1024u + 16l: the fp16 values 32u + 8q .. 32u + 8q + 7 of activation row
 //           16t + j (the f16 MFMA B operand of the slice). Slices 4h..4h+3 are 4 KB contiguous.
 //   scales  1024 B at nct * nb * 8192 + (t * nb + b) * 1024: fp32 d of (row j, slice u) at 32j + 4u
-//           (a lane reads the 4 scales of its half block with one 16-byte load); for Q4_K
-//           weights, d is the fp16-rounded scale, and 512 + 32j + 4u holds the fp16 sum of the
-//           slice's x values widened to fp32 (DS4's half2 sum), the activation side of the min
-//           term.
+//           (a lane reads the 4 scales of its half block with one 16-byte load). The activation side
+//           of the min terms follows, in bf16 pieces that add up to it exactly (the B operand of a
+//           bf16 MFMA whose A operand holds the integer mins):
+//           Q4_K: d is the fp16-rounded scale; at 512 + 32j, eight bf16 (slices 0..7) of the high
+//           pieces of the fp16 sums of the slices' x (DS4's half2 sum), at + 16 the low pieces.
+//           Q2_K (2048 B): d is the fp16-rounded scale of 64 values; for half block h at 512 + 768h +
+//           48j, + 16 and + 32: eight bf16 (16-value groups 0..7 of the half) of the first, second
+//           and third pieces of, for groups 0..5, the fp16 sum of the group's x, and for groups 6
+//           and 7 d x the sum of q (D2S6).
 constexpr int kXhUnit = 8192;       // fp16 value bytes per (column tile, K block)
-constexpr int kXhScaleUnit = 1024;  // scale bytes per (column tile, K block)
+
+// scale bytes per (column tile, K block)
+__host__ __device__ constexpr int xh_scale_unit(int type) { return type == kQ2_K ? 2048 : 1024; }
 
 __host__ __device__ inline int64_t xh_scale_base(int64_t nct, int64_t nb) { return nct * nb * kXhUnit; }
 
-__host__ __device__ inline size_t xh_bytes(int64_t n, int64_t k) {
+__host__ __device__ inline size_t xh_bytes(int64_t n, int64_t k, int type) {
   const int64_t nct = xq_col_tiles(n), nb = k / kQK;
-  return (size_t)(nct * nb * (kXhUnit + kXhScaleUnit));
+  return (size_t)(nct * nb * (kXhUnit + xh_scale_unit(type)));
 }
 
 // MFMA B operand of slice 2i + h from the 16 bytes b[t][i] of a lane's xq unit
