@@ -60,6 +60,7 @@ struct PfPlan {
   int64_t per, rem;
   int ub;         // K blocks per unit: 1, or nb where there is no room for partial sums
   int nrg;        // row groups; tile t = column group t / nrg, row group t % nrg
+  bool few;       // fewer tiles than workgroups (the numbering of the slots)
 };
 
 __device__ __forceinline__ int64_t pf_begin(const PfPlan& p, int64_t w) { return w * p.per + min(w, p.rem); }
@@ -112,7 +113,7 @@ __global__ void __launch_bounds__(kPfThreads) gemm_prefill_h_kernel(const uint8_
   using Raw = typename Dec::Raw;
   constexpr bool IQ3 = pf_iq3(TYPE);   // the unit layouts: a 16-row tile is 4 units
   constexpr bool MIN = pf_min(TYPE);   // the min term
-  constexpr int AMH = TYPE == kQ2_K ? 2048 : 1024;  // min operands of a half
+  constexpr int AMH = 2048;  // min operands of a half
   constexpr bool SUB = TYPE == kIQ4_XS;  // sub-scales applied to the dots
   constexpr bool LO = TYPE == kQ6_KX;   // two planes of operands, added in the MFMA
   constexpr int RT = kPfRowTiles / RS;  // row tiles per wave
@@ -256,7 +257,8 @@ __global__ void __launch_bounds__(kPfThreads) gemm_prefill_h_kernel(const uint8_
           f4 rt;
           if constexpr (H == 0) rt = *(const f4*)(RTs + (r0 + r) * 16 + 4 * q);
           if constexpr (MIN) {
-            const uint16_t* am = (H == 0 ? L0.AM : L1.AM) + ((r0 + r) * 16 + j) * 8;
+            const uint16_t* am = (H == 0 ? L0.AM : L1.AM) + ((r0 + r) * 16 + j) * (TYPE == kQ4_K ? 16 : 8) +
+                                 (TYPE == kQ4_K ? 8 * (q & 1) : 0);
             const f4 rm = *(const f4*)((H == 0 ? L0.RM : L1.RM) + (r0 + r) * 16 + 4 * q);
             const b8 am8 = __builtin_bit_cast(b8, *(const u32x4*)am);
 #pragma unroll
@@ -374,8 +376,11 @@ __global__ void __launch_bounds__(kPfThreads) gemm_prefill_h_kernel(const uint8_
       const int64_t first = pf_owner(plan, tile * nb);
       const int parts = (int)(pf_owner(plan, tile * nb + nb - 1) - first) + 1;
       const int mine = (int)(wg - first);
-      // slot of a workgroup's part: 2 w where the part continues a tile, 2 w + 1 where it starts one
-      auto slot_of = [&](int i) { return part + ((first + i) * 2 + (i == 0 ? 1 : 0)) * kSlot; };
+      // slot of a workgroup's part: 2 w where the part continues a tile, 2 w + 1 where it starts one; or
+      // w + tile, which grows with every part in turn
+      auto slot_of = [&](int i) {
+        return part + (plan.few ? first + i + tile : (first + i) * 2 + (i == 0 ? 1 : 0)) * kSlot;
+      };
       uint64_t* out = (uint64_t*)slot_of(mine);
 #pragma unroll
       for (int i = 0; i < RT * 2; ++i) {
@@ -467,6 +472,7 @@ void launch_prefill_h(const PfShape& s, const uint8_t* W, int64_t row_bytes, int
   PfPlan p;
   p.ub = split ? 1 : (int)nb;
   p.nrg = (nrows + 127) / 128;
+  p.few = tiles < s.wgs;
   const int64_t units = split ? tiles * nb : tiles;
   const int64_t wgs = split ? s.wgs : std::min<int64_t>(device_cus(), tiles);
   p.per = units / wgs;
@@ -496,14 +502,14 @@ bool prefill_supported(int type, bool packed) {
          type == kIQ2_S;
 }
 
-// Tile counters of the split plan, and the bytes of its partial sums (two slots per workgroup; 0: the
-// runs are whole tiles and nothing is split).
+// Tile counters of the split plan, and the bytes of its partial sums (a slot per workgroup and
+// split tile; 0: the runs are whole tiles and nothing is split).
 int64_t prefill_counters(int64_t nrows, int64_t k, int64_t n) { return pf_shape(nrows, k, n).tiles; }
 size_t prefill_slot_bytes(int64_t nrows, int64_t k, int64_t n) {
   const int64_t nb = k / kQK;
   const PfShape s = pf_shape(nrows, k, n);
   if (s.tiles * nb % s.wgs == 0 && s.tiles * nb / s.wgs % nb == 0) return 0;
-  return (size_t)(s.wgs * 2) * (16 / s.rs) * 2 * 4096;
+  return (size_t)(s.wgs + std::min(s.wgs, s.tiles)) * (16 / s.rs) * 2 * 4096;
 }
 
 // Large-M products; xh: X in the xh layout of the type; part: prefill_slot_bytes of workspace, with

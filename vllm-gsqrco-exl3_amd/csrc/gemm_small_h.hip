@@ -130,6 +130,8 @@ __global__ void __launch_bounds__(64 * (DPT * RT + NM * MW), RANGE ? 1 : 4) gemm
     // never stored). Past the end, the loads re-read block nb - 1 and the decode repeats it, which
     // leaves e and EF as they are.
     const int dt = wave / DPT;
+    int j, q;  // neighbouring lanes read neighbouring bytes
+    pf_lane(IQ3, lane, j, q);
     const int dtile = min(tile0 + dt, tile1 - 1);
     const uint8_t* wp;
     if constexpr (IQ3) wp = W + (int64_t)dtile * kTileRows * row_bytes;
@@ -226,16 +228,14 @@ __global__ void __launch_bounds__(64 * (DPT * RT + NM * MW), RANGE ? 1 : 4) gemm
   // once consumed: one step of prefetch is shorter than the load latency under this traffic
   struct BSet {
     u32x4 bq[8];
-    float dq[8], sqv[2];
+    float dq[8];
+    uint32_t sq[2];  // the two bf16 pieces of Q4_K's sums: kept as loaded, added where they are used
   };
   auto load_b = [&](BSet& o, int s, int b) {
     o.bq[s] = *(const u32x4*)(xv + (int64_t)b * kXhUnit + 1024 * s);
     o.dq[s] = *(const float*)(xs + (int64_t)b * xh_scale_unit(TYPE) + 4 * s);
     if constexpr (!IQ3)
-      if ((s & 3) == 0) {  // the two bf16 pieces of slice s + q's sum
-        const uint8_t* p = xs + (int64_t)b * xh_scale_unit(TYPE) + 512 + 2 * (s + q);
-        o.sqv[s >> 2] = __uint_as_float(ld16(p) << 16) + __uint_as_float(ld16(p + 16) << 16);
-      }
+      if ((s & 3) == 0) o.sq[s >> 2] = *(const uint32_t*)(xs + (int64_t)b * xh_scale_unit(TYPE) + 512 + 4 * (s + q));
   };
   f4 acc[TPM];
 #pragma unroll
@@ -277,10 +277,11 @@ __global__ void __launch_bounds__(64 * (DPT * RT + NM * MW), RANGE ? 1 : 4) gemm
         }
       }
       if constexpr (!IQ3) {  // the min term of the half block
+        const float sqv = __uint_as_float(o.sq[h] << 16) + __uint_as_float(o.sq[h] & 0xFFFF0000u);
 #pragma unroll
         for (int t = 0; t < TPM; ++t) {
           const float am = AM[par][h][(tix[t] * 4 + q) * 16 + j];
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(am, o.sqv[h], acc[t], 0, 0, 0);
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(am, sqv, acc[t], 0, 0, 0);
           asm volatile("" : "+v"(acc[t]));
         }
       }

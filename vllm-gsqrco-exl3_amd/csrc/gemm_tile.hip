@@ -84,10 +84,10 @@ __device__ __forceinline__ void load_xq_frag(__amdgpu_buffer_rsrc_t rs, const in
     const int unit = units[t] + b;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      x.b[t][i] = __builtin_amdgcn_raw_buffer_load_b128(rs, 64 * lane + 16 * i, unit * kXqUnit, 0);
+      x.b[t][i] = __builtin_amdgcn_raw_buffer_load_b128(rs, 16 * lane + 1024 * i, unit * kXqUnit, 0);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
-      x.d[t][i] = __builtin_amdgcn_raw_buffer_load_b128(rs, 32 * j + 16 * i, sbase + unit * kXqScaleUnit, 0);
+      x.d[t][i] = __builtin_amdgcn_raw_buffer_load_b128(rs, 16 * j + 256 * i, sbase + unit * kXqScaleUnit, 0);
   }
 }
 

@@ -25,7 +25,8 @@ struct PfLds {
   uint8_t* A;      // decoded operands of the step's half
   float* RT;       // [128] e_prev / e_cur, at block starts
   float* EF;       // [128] e_cur
-  uint16_t* AM;    // the half's mins, bf16: [tile][row][8] (Q2_K: two such planes)
+  uint16_t* AM;    // the mins, bf16: Q2_K the half's in two planes of [tile][row][8], Q4_K the
+                   // block's in [tile][row][16]
   float* RM;       // [128] -dmin / e of the half's block (Q2_K: -1 / e)
   float* LS;       // IQ4_XS: the half's sub-scales, [tile][slice][16 rows]
   const uint8_t* tbl;
@@ -39,17 +40,6 @@ struct PfLds {
 constexpr int kPfRegion = 1024;
 __device__ __forceinline__ int pf_off(int t, int u, int j, int q) {
   return (t * 4 + u) * kPfRegion + (q * 16 + (j ^ (4 * u))) * 16;
-}
-
-// decode lane -> row j of the tile and index q
-__device__ __forceinline__ void pf_lane(bool iq3, int lane, int& j, int& q) {
-  if (iq3) {  // unit lane >> 4: the 4 slices of a row pair of a unit are 64 contiguous bytes
-    j = 4 * (lane >> 4) + 2 * ((lane >> 3) & 1) + (lane & 1);
-    q = (lane >> 1) & 3;
-  } else {
-    j = lane >> 2;
-    q = lane & 3;
-  }
 }
 
 constexpr int kPfPlane = 8 * 4 * kPfRegion;  // operands of half a K block of 128 rows: 32 KB
@@ -358,7 +348,8 @@ struct PfDec<kIQ2_S> {
   }
 };
 
-// Q4_K: nibble x sc. The block's 8 mins go out with half 0 (AM: one bf16 per slice), as does RM.
+// Q4_K: nibble x sc. The block's 8 mins go out with half 0 (AM: each twice, for the two pieces of its
+// slice's sum), as does RM.
 template <>
 struct PfDec<kQ4_K> {
   struct Raw {
@@ -389,7 +380,7 @@ struct PfDec<kQ4_K> {
       sc = s0 & 0x3F3F3F3Fu;
       const uint32_t mlo = m0 & 0x3F3F3F3Fu, mhi = ((x >> 4) & 0x0F0F0F0Fu) | ((m0 >> 2) & 0x30303030u);
       const uint32_t mm = (q < 2 ? mlo : mhi) >> (16 * (q & 1));  // this lane: slices 2q, 2q + 1
-      *(uint32_t*)(s.AM + row * 8 + 2 * q) = small_bf16(mm & 0xFF) | (small_bf16((mm >> 8) & 0xFF) << 16);
+      *(uint2*)(s.AM + row * 16 + 4 * q) = make_uint2(small_bf16(mm & 0xFF) * 0x10001u, small_bf16((mm >> 8) & 0xFF) * 0x10001u);
     } else {
       sc = (x & 0x0F0F0F0Fu) | ((s0 >> 2) & 0x30303030u);
     }

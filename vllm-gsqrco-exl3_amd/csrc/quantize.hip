@@ -136,13 +136,13 @@ __device__ __forceinline__ void xq_store(uint8_t* y, int k, int c, int kk, int n
   const int u = (kk / kQ81) & 7, q = (kk / 8) & 3;
   const int t = c / kXqCols, j = c % kXqCols;
   const int64_t unit = (int64_t)t * nb + b;
-  *(uint2*)(y + unit * kXqUnit + (16 * q + j) * 64 + 8 * u) = make_uint2(lo, hi);
+  *(uint2*)(y + unit * kXqUnit + xq_value_off(16 * q + j, u)) = make_uint2(lo, hi);
   if (q == 0) {
     const uint32_t dh = __half_as_ushort(__float2half_rn(d));
     uint32_t word = VEC ? __float_as_uint(half_bits_to_float(dh)) : __float_as_uint(d);
     if constexpr (DS4)
       word = dh | (VEC ? (uint32_t)qsum << 16 : (uint32_t)__half_as_ushort(__float2half_rn(xsum)) << 16);
-    *(uint32_t*)(y + xq_scale_base(nct, nb) + (unit * kXqCols + j) * 32 + 4 * u) = word;
+    *(uint32_t*)(y + xq_scale_base(nct, nb) + unit * kXqScaleUnit + xq_scale_off(j, u)) = word;
   }
 }
 
@@ -308,7 +308,7 @@ __global__ void __launch_bounds__(256) quantize_xh_kernel(const void* __restrict
         r = fabsf(s) < INFINITY ? r - __uint_as_float(piece[z] << 16) : 0.0f;
       }
       if constexpr (LAYOUT == kDS4) {
-        if (q < 2) *(uint16_t*)(sc + 512 + 32 * j + 16 * q + 2 * u) = (uint16_t)(q == 0 ? piece[0] : piece[1]);
+        if (q == 0) *(uint32_t*)(sc + 512 + 32 * j + 4 * u) = piece[0] | (piece[1] << 16);
       } else if ((q & 1) == 0) {  // group 2 (u & 3) + (q >> 1) of half u >> 2
         uint8_t* p = sc + 512 + 768 * (u >> 2) + 48 * j + 2 * (2 * (u & 3) + (q >> 1));
 #pragma unroll

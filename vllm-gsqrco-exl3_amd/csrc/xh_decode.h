@@ -36,6 +36,17 @@ __device__ __forceinline__ int h_off(int t, int u, int j, int q) {
 __device__ __forceinline__ uint32_t h2_bits(h2 v) { return __builtin_bit_cast(uint32_t, v); }
 __device__ __forceinline__ h2 bits_h2(uint32_t v) { return __builtin_bit_cast(h2, v); }
 
+// decode lane -> row j of the tile and index q
+__device__ __forceinline__ void pf_lane(bool iq3, int lane, int& j, int& q) {
+  if (iq3) {  // unit lane >> 4: the 4 slices of a row pair of a unit are 64 contiguous bytes
+    j = 4 * (lane >> 4) + 2 * ((lane >> 3) & 1) + (lane & 1);
+    q = (lane >> 1) & 3;
+  } else {
+    j = lane >> 2;
+    q = lane & 3;
+  }
+}
+
 // A decoding lane's raw weight bytes for one step, loaded two steps ahead.
 // (16- and 8-bit loads kept narrow: a 32-bit field is widened where the loop's register sets meet,
 // at its head, which waits for every load in flight, the prefetch of the next steps included)

@@ -7,11 +7,13 @@
 // K block b (nb = K / 256 blocks):
 //   values  4096 B at ((t * nb + b) * 4096): lane l = 16q + j of a wave owns, for the block's
 //           slices u = 0..7, the eight q8 values 32u + 8q .. 32u + 8q + 7 of activation row
-//           16t + j, 8 bytes at 64l + 8u. One wave reads a (t, b) unit with four contiguous
-//           16-byte loads per lane, and those bytes are the MFMA B operands of the 8 slices.
-//   scales  512 B at nct * nb * 4096 + ((t * nb + b) * 16 + j) * 32: one dword per slice
-//           u = 0..7 of activation row 16t + j: fp32 d, or for Q4_K weights fp16 d in the low half
-//           and, above it, the activation side of Q4_K's min term: with the decode ops' q8_1
+//           16t + j, 8 bytes at 1024 (u >> 1) + 16l + 8 (u & 1). One wave reads a (t, b) unit with
+//           four 16-byte loads per lane, each a contiguous KB, and those bytes are the MFMA B
+//           operands of the 8 slices. (With a lane's 64 bytes contiguous, each load went out as 64
+//           L1 accesses instead of 16.)
+//   scales  512 B at nct * nb * 4096 + (t * nb + b) * 512: one dword per slice u = 0..7 of activation
+//           row 16t + j at 256 (u >> 2) + 16j + 4 (u & 3): fp32 d, or for Q4_K weights fp16 d in the
+//           low half and, above it, the activation side of Q4_K's min term: with the decode ops' q8_1
 //           arithmetic the slice's int16 sum of q (times d: the MMVQ form, |sum| <= 4064, exact
 //           in fp32), with the MMQ arithmetic the fp16 of the slice's sum of x (the half2 sum of
 //           block_q8_1_mmq's DS4 layout, the MMQ form, vecdotq.cuh:549-552).
@@ -30,6 +32,10 @@ constexpr int kXqScaleUnit = 512;   // scale bytes per (column tile, K block)
 
 __host__ __device__ inline int64_t xq_col_tiles(int64_t n) { return (n + kXqCols - 1) / kXqCols; }
 
+// byte offsets inside a unit: the value bytes of slice u of lane l, and (for the scales) row j's word
+__host__ __device__ constexpr int xq_value_off(int l, int u) { return 1024 * (u >> 1) + 16 * l + 8 * (u & 1); }
+__host__ __device__ constexpr int xq_scale_off(int j, int u) { return 256 * (u >> 2) + 16 * j + 4 * (u & 3); }
+
 __host__ __device__ inline int64_t xq_scale_base(int64_t nct, int64_t nb) { return nct * nb * kXqUnit; }
 
 __host__ __device__ inline size_t xq_bytes(int64_t n, int64_t k) {
@@ -46,8 +52,8 @@ __host__ __device__ inline size_t xq_bytes(int64_t n, int64_t k) {
 //           (a lane reads the 4 scales of its half block with one 16-byte load). The activation side
 //           of the min terms follows, in bf16 pieces that add up to it exactly (the B operand of a
 //           bf16 MFMA whose A operand holds the integer mins):
-//           Q4_K: d is the fp16-rounded scale; at 512 + 32j, eight bf16 (slices 0..7) of the high
-//           pieces of the fp16 sums of the slices' x (DS4's half2 sum), at + 16 the low pieces.
+//           Q4_K: d is the fp16-rounded scale; at 512 + 32j + 4u the two bf16 pieces (the first in the
+//           low half) of the fp16 sum of the slice's x (DS4's half2 sum).
 //           Q2_K (2048 B): d is the fp16-rounded scale of 64 values; for half block h at 512 + 768h +
 //           48j, + 16 and + 32: eight bf16 (16-value groups 0..7 of the half) of the first, second
 //           and third pieces of, for groups 0..5, the fp16 sum of the group's x, and for groups 6
