@@ -74,7 +74,7 @@ def test_split_and_unsplit_exact(lib, qt, rows, k, n):
     w, xg = _weight(qt, raw), x.cuda()
     assert np.array_equal(_torch_op(qt, w, xg, rows).cpu().numpy(), ref)
     y, nb = _capi_op(lib, qt, w, xg, rows)
-    assert nb == -(-n // 16) * (k // 256) * (8192 + (2048 if qt == o.Q2_K else 1024))  # the prefill GEMM's layout
+    assert nb == -(-n // 16) * (k // 256) * (8192 + (2560 if qt == o.Q2_K else 1024))  # the prefill GEMM's layout
     assert np.array_equal(y.cpu().numpy(), ref)
 
 
@@ -136,3 +136,20 @@ def test_noalloc_in_parts(lib, qt, n):
     b, _ = _capi_op(lib, qt, w, x, rows)
     # the parts' plans may add in another order: 8 fp32 roundings of sums of 160 slice terms
     assert float((a - b).norm() / b.norm()) <= 8 * 2.0 ** -24 * np.sqrt(160)
+
+
+@pytest.mark.parametrize("n", [16, 100])
+def test_q2k_group_sum_beyond_fp16(n):
+    """A 16-value group whose sum overflows fp16 (D2S6 keeps it as fp16): every weight row with a
+    nonzero min there gives dmin m's infinity, not a NaN from 0 x inf in the second plane of mins."""
+    rows, k = 400, 2560
+    raw = w_rand(o.Q2_K, rows, k, seed=7)
+    x = x_rand(n, k, seed=8, dtype=torch.float32)
+    x[1, 64:80] = -60000.0
+    y = _torch_op(o.Q2_K, dev(raw), x.cuda(), rows).cpu().numpy()
+    blk = np.ascontiguousarray(raw).reshape(rows, k // 256, 84)[:, 0]
+    dmin = np.ascontiguousarray(blk[:, 82:84]).view(np.float16)[:, 0].astype(np.float32)
+    min4 = (dmin * (blk[:, 4] >> 4)).astype(np.float16)
+    some = min4 != 0
+    assert some.any() and np.array_equal(y[1, some], np.sign(min4[some]).astype(np.float32) * np.inf)
+    assert np.isfinite(np.delete(y, 1, axis=0)).all()

@@ -281,7 +281,7 @@ bool small_fp16_shape(int op, int64_t type, int64_t k, int64_t n);
 // column tile's copy fits the static scratch.
 bool prefill_route(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
   if (!op_gemm(op) || !gguf::prefill_supported((int)type, op_packed(op))) return false;
-  if (type == gguf::kQ2_K) return gguf::xh_bytes(16, k, (int)type) <= kScratchBytes;  // K <= 209k
+  if (type == gguf::kQ2_K) return gguf::xh_bytes(16, k, (int)type) <= kScratchBytes;  // K <= 199k
   const int64_t values = row * k;
   const int64_t from = values >= (16 << 20) ? (small_fp16_shape(op, type, k, 64) ? 64 : 65) : values >= (8 << 20) ? 129 : 257;
   return n >= from;

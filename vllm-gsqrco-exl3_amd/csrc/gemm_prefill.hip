@@ -192,7 +192,7 @@ __global__ void __launch_bounds__(kPfThreads) gemm_prefill_h_kernel(const uint8_
         dxn[c] = *(const f4*)(s + 32 * j + 16 * h);
         if constexpr (TYPE == kQ4_K)
           if (h == 0) mb[c] = *(const u32x4*)(s + 512 + 32 * j + 16 * (q & 1));
-        if constexpr (TYPE == kQ2_K) mb[c] = *(const u32x4*)(s + 512 + 768 * h + 48 * j + 16 * (q < 3 ? q : 2));
+        if constexpr (TYPE == kQ2_K) mb[c] = *(const u32x4*)(s + 512 + 1024 * h + 64 * j + 16 * q);
       }
     };
     auto take_scales = [&]() {
@@ -265,9 +265,11 @@ __global__ void __launch_bounds__(kPfThreads) gemm_prefill_h_kernel(const uint8_
             for (int c = 0; c < 2; ++c) {
               const u32x4 bz = q < (TYPE == kQ4_K ? 2 : 3) ? mbc[c] : u32x4{0, 0, 0, 0};
               f4 pm = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am8, __builtin_bit_cast(b8, bz), zero, 0, 0, 0);
-              if constexpr (TYPE == kQ2_K)
+              if constexpr (TYPE == kQ2_K) {  // the mins' second pieces, on sums without infinities
+                const u32x4 bf = q > 0 ? mbc[c] : u32x4{0, 0, 0, 0};
                 pm = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, *(const u32x4*)(am + 1024)),
-                                                             __builtin_bit_cast(b8, bz), pm, 0, 0, 0);
+                                                             __builtin_bit_cast(b8, bf), pm, 0, 0, 0);
+              }
 #pragma unroll
               for (int v = 0; v < 4; ++v) {
                 if constexpr (H == 0) acc[r][c][v] *= rt[v];

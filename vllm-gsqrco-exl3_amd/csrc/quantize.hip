@@ -220,7 +220,7 @@ __global__ void __launch_bounds__(256) quantize_xh_kernel(const void* __restrict
                                                           int64_t zero_words) {
   if (zero != nullptr && blockIdx.x == 0 && blockIdx.y == 0)
     for (int64_t i = threadIdx.x; i < zero_words; i += 256) zero[i] = 0u;
-  constexpr int SU = LAYOUT == kD2S6 ? 2048 : 1024;
+  constexpr int SU = LAYOUT == kD2S6 ? 2560 : 1024;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, j = lane & 15, q = lane >> 4;
   const int nb = k / kQK, b = blockIdx.x, t = t0 + (int)blockIdx.y;
   const int c = t * kXqCols + j;
@@ -310,9 +310,10 @@ __global__ void __launch_bounds__(256) quantize_xh_kernel(const void* __restrict
       if constexpr (LAYOUT == kDS4) {
         if (q == 0) *(uint32_t*)(sc + 512 + 32 * j + 4 * u) = piece[0] | (piece[1] << 16);
       } else if ((q & 1) == 0) {  // group 2 (u & 3) + (q >> 1) of half u >> 2
-        uint8_t* p = sc + 512 + 768 * (u >> 2) + 48 * j + 2 * (2 * (u & 3) + (q >> 1));
+        uint8_t* p = sc + 512 + 1024 * (u >> 2) + 64 * j + 2 * (2 * (u & 3) + (q >> 1));
 #pragma unroll
         for (int z = 0; z < 3; ++z) *(uint16_t*)(p + 16 * z) = (uint16_t)piece[z];
+        *(uint16_t*)(p + 48) = fabsf(s) < INFINITY ? (uint16_t)piece[0] : 0;
       }
     }
   }

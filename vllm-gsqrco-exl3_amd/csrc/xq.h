@@ -54,14 +54,15 @@ __host__ __device__ inline size_t xq_bytes(int64_t n, int64_t k) {
 //           bf16 MFMA whose A operand holds the integer mins):
 //           Q4_K: d is the fp16-rounded scale; at 512 + 32j + 4u the two bf16 pieces (the first in the
 //           low half) of the fp16 sum of the slice's x (DS4's half2 sum).
-//           Q2_K (2048 B): d is the fp16-rounded scale of 64 values; for half block h at 512 + 768h +
-//           48j, + 16 and + 32: eight bf16 (16-value groups 0..7 of the half) of the first, second
+//           Q2_K (2560 B): d is the fp16-rounded scale of 64 values; for half block h at 512 + 1024h +
+//           64j, + 16 and + 32: eight bf16 (16-value groups 0..7 of the half) of the first, second
 //           and third pieces of, for groups 0..5, the fp16 sum of the group's x, and for groups 6
-//           and 7 d x the sum of q (D2S6).
+//           and 7 d x the sum of q (D2S6); at + 48 the first piece again, 0 where the sum is not
+//           finite (the operand of the mins' second pieces: 0 x inf would make a NaN of an inf).
 constexpr int kXhUnit = 8192;       // fp16 value bytes per (column tile, K block)
 
 // scale bytes per (column tile, K block)
-__host__ __device__ constexpr int xh_scale_unit(int type) { return type == kQ2_K ? 2048 : 1024; }
+__host__ __device__ constexpr int xh_scale_unit(int type) { return type == kQ2_K ? 2560 : 1024; }
 
 __host__ __device__ inline int64_t xh_scale_base(int64_t nct, int64_t nb) { return nct * nb * kXhUnit; }
 
