@@ -153,3 +153,26 @@ def test_q2k_group_sum_beyond_fp16(n):
     some = min4 != 0
     assert some.any() and np.array_equal(y[1, some], np.sign(min4[some]).astype(np.float32) * np.inf)
     assert np.isfinite(np.delete(y, 1, axis=0)).all()
+
+
+# (270, 2560, 24) and (270, 2560, 300): 64-column tiles; (4102, 2560, 600): 128; (16390, 2560, 1000): 256
+@pytest.mark.parametrize("rows,k,n", [(270, 2560, 24), (270, 2560, 300), (4102, 2560, 600), (16390, 2560, 1000)])
+@pytest.mark.parametrize("scales", ["ordinary", "subnormal", "wide"])
+def test_q2k_scales_rounded_as_the_model(rows, k, n, scales):
+    """Q2_K's products keep d times sub-scale as fp16, as the reference's tile loader does: fp32 X against
+    the float64 model that rounds there. The rest is fp32 sums: 2^-24 of the partial sum at each of the
+    K / 32 slices, adding up at random. (An unrounded d times sub-scale is 2.5e-4 off.) Scales of an
+    ordinary file, of which many are fp16 subnormals, and from 2^-20 to 2^10 within a row with zeros
+    among them, for which the rows' unit of account moves."""
+    raw = o.random_blocks(np.random.default_rng(n), o.Q2_K, rows, k, scale_sigma=3e-6 if scales == "subnormal" else 2e-3)
+    if scales == "wide":
+        rng = np.random.default_rng(n + 1)
+        b = raw.reshape(-1, 84)
+        for at in o.SCALE_OFFSETS[o.Q2_K]:
+            d = (2.0 ** rng.uniform(-20, 10, len(b)) * (rng.random(len(b)) > 0.1)).astype(np.float16)
+            b[:, at:at + 2] = d.view(np.uint8).reshape(-1, 2)
+    x = x_rand(n, k, seed=n + 2)
+    y = _torch_op(o.Q2_K, dev(raw), x.cuda(), rows).cpu().numpy()
+    rs = np.unique(np.random.default_rng(3).choice(rows, 64, replace=False))
+    ref = o.q81_model(raw[rs], o.Q2_K, x, layout="mmq")
+    assert o.rel_l2(y[:, rs], ref) <= 2 * np.sqrt(k / 32) * 2.0 ** -24

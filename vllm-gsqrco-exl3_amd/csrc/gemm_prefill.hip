@@ -14,7 +14,13 @@
 // a new block starts and by the last e at the end. The min term of Q4_K, sum over slices of (-dmin / e)
 // m_g s_g, is an integer-weighted sum of the activation sums s_g: one bf16 MFMA per block over m_g
 // (exact in bf16) and s_g in bf16 pieces that add up to it exactly, then one FMA per output by -dmin /
-// e. Q2_K's, over 16-value groups with the fp16 of dmin m_g, is two per half block (two pieces of it).
+// e. Q2_K rounds d times its sub-scale to fp16 (f), so its operands are f (q - 1) in units of a power of
+// two and the slices are no integers: the two slices of 64 values, which share an activation scale, and
+// the sum f x (sum of q8) that makes up for the - 1 are one chain of three MFMAs (one for f of 4 groups),
+// one FMA per output and chain; its mins, over 16-value groups with the fp16 of dmin m_g, are two bf16
+// MFMAs per half block (two pieces of it) onto the accumulator. 12288 x 5120, M = 24 / 512 / 1024: 44 / 140
+// / 260 us; with 3f rounded off into a second plane of operands, five MFMAs per 64 values and column, 48 /
+// 191 / 358; with d left outside (f not rounded) 40 / 132 / 253.
 //
 // Workgroup: 8 waves over 128 weight rows x 256 / RS activation rows. Wave w owns 2 column tiles of
 // 16 and 8 / RS of the 8 row tiles (RS row parts share a column pair). Its B operands come straight
@@ -113,24 +119,28 @@ __global__ void __launch_bounds__(kPfThreads) gemm_prefill_h_kernel(const uint8_
   using Raw = typename Dec::Raw;
   constexpr bool IQ3 = pf_iq3(TYPE);   // the unit layouts: a 16-row tile is 4 units
   constexpr bool MIN = pf_min(TYPE);   // the min term
-  constexpr int AMH = 2048;  // min operands of a half
+  constexpr int AMH = TYPE == kQ2_K ? 5120 : 2048;  // min operands of a half
   constexpr bool SUB = TYPE == kIQ4_XS;  // sub-scales applied to the dots
   constexpr bool LO = TYPE == kQ6_KX;   // two planes of operands, added in the MFMA
+  // slices 2i, 2i + 1 in one chain of MFMAs: they share an activation scale (D2S6); the chain ends with
+  // the sum that the operands' offset needs (pf_decode.h)
+  constexpr bool PAIR = TYPE == kQ2_K;
   constexpr int RT = kPfRowTiles / RS;  // row tiles per wave
   constexpr int CG = kPfWaves / RS;     // column pairs per workgroup
   // row tiles per MFMA group: 4 MFMAs and their 16 FMAs in a row beat 2 and 8 by 3 %; with sub-scales
   // or two planes two row tiles' operands spill
-  constexpr int GR = SUB || LO ? 1 : 2;
-  constexpr int NG = RT / GR;           // groups per slice
-  constexpr int AD = GR == 1 ? 2 : 1;   // groups ahead that A operands are read
+  constexpr int GR = SUB || LO || PAIR ? 1 : 2;
+  constexpr int NG = RT / GR;           // groups per slice (PAIR: per two slices)
+  constexpr int GS = PAIR ? 2 : 4;      // groups of NG per step
+  constexpr int AD = GR == 1 && !PAIR ? 2 : 1;  // groups ahead that A operands are read
   constexpr int BD = RS == 1 ? 1 : 2;   // steps ahead that B operands are loaded
   constexpr int SU = xh_scale_unit(TYPE);
   constexpr int TB = pf_table_bytes(TYPE);
   constexpr int kPfA = (LO ? 2 : 1) * kPfPlane;  // operands of a step
   __shared__ __attribute__((aligned(16))) uint8_t A[2 * kPfA];
-  __shared__ __attribute__((aligned(16))) float RTs[128];
+  __shared__ __attribute__((aligned(16))) float RTs[128 + kPfRowTiles];
   __shared__ __attribute__((aligned(16))) float EFs[128];
-  __shared__ __attribute__((aligned(16))) float RMs[MIN ? 256 : 4];
+  __shared__ __attribute__((aligned(16))) float RMs[TYPE == kQ4_K ? 128 : 4];
   __shared__ __attribute__((aligned(16))) uint16_t AMs[MIN ? 2 * AMH : 8];
   __shared__ __attribute__((aligned(16))) float LSs[SUB ? 2 * 512 : 4];
   __shared__ __attribute__((aligned(16))) uint4 tbl[TB ? TB / 16 : 1];
@@ -151,7 +161,7 @@ __global__ void __launch_bounds__(kPfThreads) gemm_prefill_h_kernel(const uint8_
     for (int i = threadIdx.x; i < TB / 16; i += kPfThreads) tbl[i] = src[i];
   }
   const PfLds L0 = {A, RTs, EFs, AMs, RMs, LSs, (const uint8_t*)tbl};
-  const PfLds L1 = {A + kPfA, RTs, EFs, AMs + (MIN ? AMH : 0), RMs + (MIN ? 128 : 0), LSs + (SUB ? 512 : 0),
+  const PfLds L1 = {A + kPfA, RTs, EFs, AMs + (MIN ? AMH : 0), RMs, LSs + (SUB ? 512 : 0),
                     (const uint8_t*)tbl};
 
   // consecutive workgroups go round the 8 XCDs: give each XCD a contiguous range of units, so that
@@ -235,7 +245,8 @@ __global__ void __launch_bounds__(kPfThreads) gemm_prefill_h_kernel(const uint8_
       f4 ls[AD + 1][GR];
       f4 p[GR][2];
       auto read_a = [&](int g) {
-        const int u = g / NG, r = g % NG * GR;
+        const int u = g / NG * (4 / GS), r = g % NG * GR;
+        if constexpr (PAIR) al[g % (AD + 1)][0] = *(const h8*)(Ab + pf_off(r0 + r, u + 1, j, q));
 #pragma unroll
         for (int i = 0; i < GR; ++i) {
           a[g % (AD + 1)][i] = *(const h8*)(Ab + pf_off(r0 + r + i, u, j, q));
@@ -251,28 +262,35 @@ __global__ void __launch_bounds__(kPfThreads) gemm_prefill_h_kernel(const uint8_
       __builtin_amdgcn_sched_barrier(0);
       Dec::begin(raw, ctx, HN, e, LN, wave, dj, dq);
       Dec::template issue<0>(ctx, tmp[0], LN);
-      if (H == 0 || TYPE == kQ2_K) {  // a new block: rescale every row to its e; the min term
+      // a new block: rescale the rows to its e; the min term
+      if constexpr (PAIR) {
+        // the mins' first pieces on all three pieces of the sums (q = 0, 1, 2), their second ones on the
+        // first two
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
-          f4 rt;
-          if constexpr (H == 0) rt = *(const f4*)(RTs + (r0 + r) * 16 + 4 * q);
+          const uint16_t* am = (H == 0 ? L0.AM : L1.AM) + ((r0 + r) * 16 + j) * 8;
+          const b8 hi = __builtin_bit_cast(b8, *(const u32x4*)am), lo = __builtin_bit_cast(b8, *(const u32x4*)(am + 1024));
+#pragma unroll
+          for (int c = 0; c < 2; ++c) {
+            const u32x4 b3 = q < 3 ? mbc[c] : u32x4{0, 0, 0, 0}, b2 = q < 2 ? mbc[c] : u32x4{0, 0, 0, 0};
+            acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, __builtin_bit_cast(b8, b3), acc[r][c], 0, 0, 0);
+            acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo, __builtin_bit_cast(b8, b2), acc[r][c], 0, 0, 0);
+          }
+        }
+      } else if constexpr (H == 0) {
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+          const f4 rt = *(const f4*)(RTs + (r0 + r) * 16 + 4 * q);
           if constexpr (MIN) {
-            const uint16_t* am = (H == 0 ? L0.AM : L1.AM) + ((r0 + r) * 16 + j) * (TYPE == kQ4_K ? 16 : 8) +
-                                 (TYPE == kQ4_K ? 8 * (q & 1) : 0);
-            const f4 rm = *(const f4*)((H == 0 ? L0.RM : L1.RM) + (r0 + r) * 16 + 4 * q);
-            const b8 am8 = __builtin_bit_cast(b8, *(const u32x4*)am);
+            const f4 rm = *(const f4*)(RMs + (r0 + r) * 16 + 4 * q);
+            const b8 am8 = __builtin_bit_cast(b8, *(const u32x4*)(AMs + ((r0 + r) * 16 + j) * 16 + 8 * (q & 1)));
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
-              const u32x4 bz = q < (TYPE == kQ4_K ? 2 : 3) ? mbc[c] : u32x4{0, 0, 0, 0};
-              f4 pm = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am8, __builtin_bit_cast(b8, bz), zero, 0, 0, 0);
-              if constexpr (TYPE == kQ2_K) {  // the mins' second pieces, on sums without infinities
-                const u32x4 bf = q > 0 ? mbc[c] : u32x4{0, 0, 0, 0};
-                pm = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, *(const u32x4*)(am + 1024)),
-                                                             __builtin_bit_cast(b8, bf), pm, 0, 0, 0);
-              }
+              const u32x4 bz = q < 2 ? mbc[c] : u32x4{0, 0, 0, 0};
+              const f4 pm = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am8, __builtin_bit_cast(b8, bz), zero, 0, 0, 0);
 #pragma unroll
               for (int v = 0; v < 4; ++v) {
-                if constexpr (H == 0) acc[r][c][v] *= rt[v];
+                acc[r][c][v] *= rt[v];
                 acc[r][c][v] = fmaf(pm[v], rm[v], acc[r][c][v]);
               }
             }
@@ -282,11 +300,17 @@ __global__ void __launch_bounds__(kPfThreads) gemm_prefill_h_kernel(const uint8_
           }
         }
       }
+      if constexpr (PAIR) {  // of mbc the chains use what lanes q == 3 hold
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) mbc[c][i] = q == 3 ? mbc[c][i] : 0;
+      }
       __builtin_amdgcn_sched_barrier(0);
       // group g = (slice, GR row tiles): the A operands AD groups on are read, 2 GR MFMAs issued, and
       // the previous group's results folded into acc
       auto fold = [&](int g, const f4 (&lg)[GR]) {
-        const int u = g / NG, r = g % NG * GR;
+        const int u = g / NG * (4 / GS), r = g % NG * GR;
 #pragma unroll
         for (int i = 0; i < GR; ++i)
 #pragma unroll
@@ -299,18 +323,23 @@ __global__ void __launch_bounds__(kPfThreads) gemm_prefill_h_kernel(const uint8_
       };
 #define GGUF_PF_SLICE(U)                                                                                              \
   if constexpr (U < 3) Dec::template issue<(U < 3 ? U + 1 : 3)>(ctx, tmp[(U + 1) & 1], LN);                           \
-  _Pragma("unroll") for (int gr = 0; gr < NG; ++gr) {                                                                 \
-    const int g = U * NG + gr;                                                                                        \
+  if constexpr (!PAIR || (U & 1) == 0) _Pragma("unroll") for (int gr = 0; gr < NG; ++gr) {                            \
+    const int g = U * GS / 4 * NG + gr;                                                                               \
     f4 nx[GR][2], lg[GR];                                                                                             \
     if constexpr (SUB) _Pragma("unroll") for (int i = 0; i < GR; ++i) lg[i] = ls[(g + AD) % (AD + 1)][i];             \
-    if (GR > 1 && g + AD < 4 * NG) read_a(g + AD);                                                                    \
+    if ((GR > 1 || PAIR) && g + AD < GS * NG) read_a(g + AD);                                                         \
+    h8 af;                                                                                                            \
+    if constexpr (PAIR) af = *(const h8*)((H == 0 ? L0.AM : L1.AM) + 3072 + 512 * U + ((r0 + gr) * 16 + j) * 8);      \
     _Pragma("unroll") for (int i = 0; i < GR; ++i) _Pragma("unroll") for (int c = 0; c < 2; ++c) nx[i][c] =           \
         __builtin_amdgcn_mfma_f32_16x16x32_f16(a[g % (AD + 1)][i], __builtin_bit_cast(h8, bq[c][U]), zero, 0, 0, 0);  \
-    if constexpr (LO) _Pragma("unroll") for (int i = 0; i < GR; ++i) _Pragma("unroll") for (int c = 0; c < 2; ++c)    \
-        nx[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[g % (AD + 1)][i], __builtin_bit_cast(h8, bq[c][U]),      \
-                                                          nx[i][c], 0, 0, 0);                                         \
+    if constexpr (LO || PAIR) _Pragma("unroll") for (int i = 0; i < GR; ++i) _Pragma("unroll") for (int c = 0; c < 2; \
+                                                                                                    ++c)              \
+        nx[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(                                                            \
+            al[g % (AD + 1)][i], __builtin_bit_cast(h8, bq[c][PAIR ? U | 1 : U]), nx[i][c], 0, 0, 0);                 \
+    if constexpr (PAIR) _Pragma("unroll") for (int c = 0; c < 2; ++c) nx[0][c] =                                      \
+        __builtin_amdgcn_mfma_f32_16x16x32_f16(af, __builtin_bit_cast(h8, mbc[c]), nx[0][c], 0, 0, 0);                \
     if (g > 0) fold(g - 1, lg);                                                                                       \
-    if (GR == 1 && g + AD < 4 * NG) read_a(g + AD);                                                                   \
+    if (GR == 1 && !PAIR && g + AD < GS * NG) read_a(g + AD);                                                         \
     _Pragma("unroll") for (int i = 0; i < GR; ++i) _Pragma("unroll") for (int c = 0; c < 2; ++c) p[i][c] = nx[i][c];  \
     __builtin_amdgcn_sched_barrier(0);                                                                                \
   }                                                                                                                   \
@@ -325,7 +354,7 @@ __global__ void __launch_bounds__(kPfThreads) gemm_prefill_h_kernel(const uint8_
 #undef GGUF_PF_SLICE
       // last, so that no wait for B operands or scales waits for it: loads return in order
       Dec::load(raw, wp, row_bytes, nb, braw, HN, dj, dq);
-      fold(4 * NG - 1, ls[(4 * NG - 1) % (AD + 1)]);
+      fold(GS * NG - 1, ls[(GS * NG - 1) % (AD + 1)]);
       take_scales();
     };
 
@@ -365,6 +394,16 @@ __global__ void __launch_bounds__(kPfThreads) gemm_prefill_h_kernel(const uint8_
       lds_barrier();
       step(std::integral_constant<int, 1>{}, bn, raw0, bn, min(b + 2, b1 - 1));
       lds_barrier();
+      if constexpr (PAIR) {  // the rows' e has moved: hardly ever
+        if (__any(RTs[128 + (lane & 7)] != 0.0f)) {
+#pragma unroll
+          for (int r = 0; r < RT; ++r) {
+            const f4 rt = *(const f4*)(RTs + (r0 + r) * 16 + 4 * q);
+            acc[r][0] *= rt;
+            acc[r][1] *= rt;
+          }
+        }
+      }
     }
 #pragma unroll
     for (int r = 0; r < RT; ++r) {

@@ -8,9 +8,10 @@
 // so that neighbours read neighbouring bytes (pf_lane): the loads of a tile's rows by lane = 16 q + j
 // went out as nearly one L1 access per lane, 2400 of the 3560 a step of a workgroup made.
 // The operand is the weight value times its sub-scale, an integer that fp16 holds exactly (IQ3_S
-// <= 465, IQ3_XXS <= 1922, IQ2 <= 1333, Q4_K <= 945, Q2_K <= 45; Q6_K's (q - 32) * sc is exact up to
-// 2048 and rounds to an even neighbour beyond, 2^-12, unless kQ6_KX keeps the rest), except IQ4_XS: codebook value x sub-scale
-// reaches 4064, so its operand is the codebook value and the sub-scale multiplies the slice's dot.
+// <= 465, IQ3_XXS <= 1922, IQ2 <= 1333, Q4_K <= 945; Q6_K's (q - 32) * sc is exact up to 2048 and rounds to
+// an even neighbour beyond, 2^-12, unless kQ6_KX keeps the rest), except IQ4_XS: codebook value x sub-scale
+// reaches 4064, so its operand is the codebook value and the sub-scale multiplies the slice's dot; and
+// Q2_K, see there.
 // The row's block scale (d; d / 8 for the IQ2 types, d / 4 for IQ3_XXS) stays outside, see next_scale.
 #pragma once
 
@@ -25,9 +26,9 @@ struct PfLds {
   uint8_t* A;      // decoded operands of the step's half
   float* RT;       // [128] e_prev / e_cur, at block starts
   float* EF;       // [128] e_cur
-  uint16_t* AM;    // the mins, bf16: Q2_K the half's in two planes of [tile][row][8], Q4_K the
-                   // block's in [tile][row][16]
-  float* RM;       // [128] -dmin / e of the half's block (Q2_K: -1 / e)
+  uint16_t* AM;    // the mins, bf16: Q2_K the half's in planes of [tile][row][8], Q4_K the block's in
+                   // [tile][row][16]
+  float* RM;       // Q4_K: [128] -dmin / e of the block
   float* LS;       // IQ4_XS: the half's sub-scales, [tile][slice][16 rows]
   const uint8_t* tbl;
 };
@@ -405,9 +406,17 @@ struct PfDec<kQ4_K> {
   }
 };
 
-// Q2_K: 2-bit quant x sc per 16 values. Each half's 8 mins go out with the half: the fp16 of dmin * m, as
-// the reference's MMQ tile loader stores it (mmq-load-tiles.cuh:582-591), in two bf16 pieces (AM, AM +
-// 1024), with RM = -1 / e. The loader also rounds d * sc to fp16; here the product stays exact.
+// 1 / v of a power of two
+__device__ __forceinline__ float pow2_inv(float v) { return __uint_as_float(0x7F000000u - __float_as_uint(v)); }
+
+// Q2_K: 2-bit quant x f, the fp16 of d * sc, per 16 values, as the reference's MMQ tile loader rounds it
+// (mmq-load-tiles.cuh:582-591). 3f may need two bits more than fp16 has, so the operand is f (q - 1), -f
+// .. 2f, and the sum f x (sum of the group's q8) that it leaves out is an MFMA of its own per 64 values
+// (f: AM + 3072 and AM + 4096, fp16, for groups 0..3 and 4..7 of the half, 0 for the others). Operands are
+// in units of e, a power of two within 2^8 of d, so that f is exact there, and so are the mins: each half's
+// 8 go out with the half, minus the fp16 of dmin * m (rounded there as well) in two bf16 pieces (AM, AM +
+// 1024). e moves only when a block's d leaves that range; the rows' accumulators are rescaled only then
+// (RT, with a flag per row tile at RT + 128).
 template <>
 struct PfDec<kQ2_K> {
   struct Raw {
@@ -416,7 +425,7 @@ struct PfDec<kQ2_K> {
     uint32_t dm;
   };
   struct Ctx {
-    h2 mul[2], off[2];
+    h2 mul[2];
     u32x4 v0, v1;
   };
   struct Tmp {};
@@ -432,25 +441,33 @@ struct PfDec<kQ2_K> {
                                                int q) {
     const float d = half_bits_to_float(w.dm & 0xFFFF);
     const int row = t * 16 + j;
-    const bool nz = d != 0.0f;
-    if (h == 0) next_scale(d, e, s.RT, s.EF, row);
-    s.RM[row] = -1.0f / e;
+    if (h == 0) {
+      // the power of two of d, for an infinite one that of the largest fp16 (no short circuit: a branch
+      // here made the step spill 140 registers)
+      const uint32_t p = min(__float_as_uint(d) & 0x7F800000u, 0x47000000u);
+      const bool move = (d != 0.0f) & (p - __float_as_uint(e) + (8u << 23) > (16u << 23));
+      const float en = move ? __uint_as_float(p) : e;
+      s.RT[row] = e * pow2_inv(en);
+      s.EF[row] = en;
+      s.RT[128 + t] = __any(en != e) ? 1.0f : 0.0f;
+      e = en;
+    }
+    const float re = pow2_inv(e);
     const uint32_t mine = (q < 2 ? w.sc.x : w.sc.y) >> (16 * (q & 1));  // groups 2q, 2q + 1: slice q's
     const float dmin = half_bits_to_float(w.dm >> 16);
     uint32_t hi[2], lo[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      const float f = __half2float(__float2half_rn(dmin * (float)((mine >> (8 * i + 4)) & 0xF)));
+      c.mul[i] = h2_of(__half2float(__float2half_rn(d * (float)((mine >> (8 * i)) & 0xF))) * re);
+      const float f = __half2float(__float2half_rn(dmin * (float)((mine >> (8 * i + 4)) & 0xF))) * -re;
       hi[i] = __float_as_uint(f) >> 16;  // the upper 8 bits of 11
       const float r = f - __uint_as_float(hi[i] << 16);
       lo[i] = __float_as_uint(r == r ? r : 0.0f) >> 16;
     }
     *(uint32_t*)(s.AM + row * 8 + 2 * q) = hi[0] | (hi[1] << 16);
     *(uint32_t*)(s.AM + 1024 + row * 8 + 2 * q) = lo[0] | (lo[1] << 16);
-    c.mul[0] = h2_of(nz ? (float)(mine & 0xF) : 0.0f);
-    c.mul[1] = h2_of(nz ? (float)((mine >> 8) & 0xF) : 0.0f);
-    c.off[0] = c.mul[0] * (_Float16)(-1024.0f);
-    c.off[1] = c.mul[1] * (_Float16)(-1024.0f);
+    *(uint32_t*)(s.AM + 3072 + 1024 * (q >> 1) + row * 8 + 2 * q) = h2_bits(h2{c.mul[0][0], c.mul[1][0]});
+    *(uint32_t*)(s.AM + 4096 - 1024 * (q >> 1) + row * 8 + 2 * q) = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       c.v0[i] = (w.v0[i] >> (2 * q)) & 0x03030303u;
@@ -462,9 +479,12 @@ struct PfDec<kQ2_K> {
   template <int I>
   __device__ __forceinline__ static void finish(const Ctx& c, const Tmp&, const PfLds& s, int t, int j, int q) {
     const u32x4 vv = I < 2 ? c.v0 : c.v1;
+    const h2 bias = {(_Float16)-1025.0f, (_Float16)-1025.0f};
     uint32_t v[4];
-    bytes_to_h4(vv[2 * (I & 1)], c.mul[I >> 1], c.off[I >> 1], v[0], v[1]);
-    bytes_to_h4(vv[2 * (I & 1) + 1], c.mul[I >> 1], c.off[I >> 1], v[2], v[3]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      v[i] = h2_bits((bits_h2(__builtin_amdgcn_perm(0x64646464u, vv[2 * (I & 1) + (i >> 1)],
+                                                    (i & 1) ? 0x04030402u : 0x04010400u)) + bias) * c.mul[I >> 1]);
     *(uint4*)(s.A + pf_off(t, q, j, I)) = make_uint4(v[0], v[1], v[2], v[3]);
   }
 };

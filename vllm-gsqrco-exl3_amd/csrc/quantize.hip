@@ -292,20 +292,25 @@ __global__ void __launch_bounds__(256) quantize_xh_kernel(const void* __restrict
       a += __shfl_xor(a, 16, 64);
       bb += __shfl_xor(bb, 16, 64);
       float s = half_bits_to_float(__half_as_ushort(__float2half_rn(a + bb)));
+      int sq = 0;
       if constexpr (LAYOUT == kD2S6) {
-        int sq = 0;
 #pragma unroll
         for (int e = 0; e < 8; ++e) sq += qv[e];
         sq += __shfl_xor(sq, 16, 64);
         if ((u & 3) == 3) s = d * (float)sq;  // groups 6, 7 of each 128 values; exact
       }
       // bf16 pieces, exact: 8 + 8 bits hold an fp16, 8 + 8 + 8 an fp32
+      const bool fin = fabsf(s) < INFINITY;
       uint32_t piece[3];
       float r = s;
 #pragma unroll
       for (int z = 0; z < 3; ++z) {
         piece[z] = f32_to_bf16_bits(r);
-        r = fabsf(s) < INFINITY ? r - __uint_as_float(piece[z] << 16) : 0.0f;
+        r = fin ? r - __uint_as_float(piece[z] << 16) : 0.0f;
+      }
+      if (LAYOUT == kD2S6 && !fin) {  // in the third place, which meets the mins' first pieces only
+        piece[2] = piece[0];
+        piece[0] = f32_to_bf16_bits(copysignf(1.0f, s));
       }
       if constexpr (LAYOUT == kDS4) {
         if (q == 0) *(uint32_t*)(sc + 512 + 32 * j + 4 * u) = piece[0] | (piece[1] << 16);
@@ -313,7 +318,7 @@ __global__ void __launch_bounds__(256) quantize_xh_kernel(const void* __restrict
         uint8_t* p = sc + 512 + 1024 * (u >> 2) + 64 * j + 2 * (2 * (u & 3) + (q >> 1));
 #pragma unroll
         for (int z = 0; z < 3; ++z) *(uint16_t*)(p + 16 * z) = (uint16_t)piece[z];
-        *(uint16_t*)(p + 48) = fabsf(s) < INFINITY ? (uint16_t)piece[0] : 0;
+        *(uint16_t*)(p + 48) = __half_as_ushort(__float2half_rn((float)sq));  // exact
       }
     }
   }

@@ -57,8 +57,9 @@ __host__ __device__ inline size_t xq_bytes(int64_t n, int64_t k) {
 //           Q2_K (2560 B): d is the fp16-rounded scale of 64 values; for half block h at 512 + 1024h +
 //           64j, + 16 and + 32: eight bf16 (16-value groups 0..7 of the half) of the first, second
 //           and third pieces of, for groups 0..5, the fp16 sum of the group's x, and for groups 6
-//           and 7 d x the sum of q (D2S6); at + 48 the first piece again, 0 where the sum is not
-//           finite (the operand of the mins' second pieces: 0 x inf would make a NaN of an inf).
+//           and 7 d x the sum of q (D2S6), with a sum that is not finite in the third place beside
+//           +-1, 0 (the mins' second pieces, often 0, meet the first two places only: 0 x inf would
+//           make a NaN of an inf); at + 48 the eight sums of q, as fp16 (exact).
 constexpr int kXhUnit = 8192;       // fp16 value bytes per (column tile, K block)
 
 // scale bytes per (column tile, K block)
