@@ -176,3 +176,28 @@ def test_q2k_scales_rounded_as_the_model(rows, k, n, scales):
     rs = np.unique(np.random.default_rng(3).choice(rows, 64, replace=False))
     ref = o.q81_model(raw[rs], o.Q2_K, x, layout="mmq")
     assert o.rel_l2(y[:, rs], ref) <= 2 * np.sqrt(k / 32) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("n", [16, 100])
+@pytest.mark.parametrize("group", [3, 6, 13, 15])
+def test_q2k_min_beyond_fp16(n, group):
+    """A min that overflows fp16 (dmin * m as the tile loader keeps it) of a group whose sum is stored
+    (0..5 of each 128 values) or taken from q8 (6, 7): the weight row's outputs are minus the sum's
+    infinity; the other rows stay finite."""
+    rows, k = 144, 1024
+    raw = w_rand(o.Q2_K, rows, k, seed=9)
+    blk = raw.reshape(rows, k // 256, 84)
+    bad = np.arange(0, rows, 7)
+    blk[bad, 1, :16] = (blk[bad, 1, :16] & 0xF) | 0x10
+    blk[bad, 1, group] |= 0xF0
+    blk[bad, 1, 82:84] = np.array([30000], np.float16).view(np.uint8)  # m = 1: finite, 15: 450000
+    x = x_rand(n, k, seed=10)
+    y = _torch_op(o.Q2_K, dev(raw), x.cuda(), rows).cpu().numpy()
+    q8 = o.quantize_q8_1_mmq(x, o.Q2_K)
+    q, _ = o.dequant_q8_1_mmq(q8, n, k, o.Q2_K)
+    sums = o.mmq_d2s6_sums(q8, n, k).reshape(n, k // 16)
+    sums = np.where(np.isnan(sums), q.astype(np.int64).reshape(n, k // 16, 16).sum(-1), sums)[:, 16 + group]
+    want = np.where(sums == 0, np.nan, -np.sign(sums) * np.inf).astype(np.float32)
+    assert (sums > 0).any() and (sums < 0).any()
+    assert np.array_equal(y[:, bad], np.repeat(want[:, None], len(bad), 1), equal_nan=True)
+    assert np.isfinite(np.delete(y, bad, axis=1)).all()

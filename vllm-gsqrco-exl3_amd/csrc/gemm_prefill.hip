@@ -18,9 +18,9 @@
 // two and the slices are no integers: the two slices of 64 values, which share an activation scale, and
 // the sum f x (sum of q8) that makes up for the - 1 are one chain of three MFMAs (one for f of 4 groups),
 // one FMA per output and chain; its mins, over 16-value groups with the fp16 of dmin m_g, are two bf16
-// MFMAs per half block (two pieces of it) onto the accumulator. 12288 x 5120, M = 24 / 512 / 1024: 44 / 140
-// / 260 us; with 3f rounded off into a second plane of operands, five MFMAs per 64 values and column, 48 /
-// 191 / 358; with d left outside (f not rounded) 40 / 132 / 253.
+// MFMAs per half block (two pieces of it) onto the accumulator. 12288 x 5120, M = 24 / 512 / 1024: 44 / 133
+// / 248 us; with 3f rounded off into a second plane of operands, four MFMAs per 64 values, 48 / 191 /
+// 358; with d left outside (f not rounded) 40 / 132 / 253.
 //
 // Workgroup: 8 waves over 128 weight rows x 256 / RS activation rows. Wave w owns 2 column tiles of
 // 16 and 8 / RS of the 8 row tiles (RS row parts share a column pair). Its B operands come straight
@@ -265,11 +265,13 @@ __global__ void __launch_bounds__(kPfThreads) gemm_prefill_h_kernel(const uint8_
       // a new block: rescale the rows to its e; the min term
       if constexpr (PAIR) {
         // the mins' first pieces on all three pieces of the sums (q = 0, 1, 2), their second ones on the
-        // first two
+        // first two; an infinite min meets the first piece only, which is 0 where the sum is (0 x inf
+        // elsewhere would make a NaN of an inf)
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
           const uint16_t* am = (H == 0 ? L0.AM : L1.AM) + ((r0 + r) * 16 + j) * 8;
-          const b8 hi = __builtin_bit_cast(b8, *(const u32x4*)am), lo = __builtin_bit_cast(b8, *(const u32x4*)(am + 1024));
+          const b8 hi = __builtin_bit_cast(b8, *(const u32x4*)(am + (q == 0 ? 0 : 2048))),
+                   lo = __builtin_bit_cast(b8, *(const u32x4*)(am + 1024));
 #pragma unroll
           for (int c = 0; c < 2; ++c) {
             const u32x4 b3 = q < 3 ? mbc[c] : u32x4{0, 0, 0, 0}, b2 = q < 2 ? mbc[c] : u32x4{0, 0, 0, 0};

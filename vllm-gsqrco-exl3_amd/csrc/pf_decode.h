@@ -415,7 +415,7 @@ __device__ __forceinline__ float pow2_inv(float v) { return __uint_as_float(0x7F
 // (f: AM + 3072 and AM + 4096, fp16, for groups 0..3 and 4..7 of the half, 0 for the others). Operands are
 // in units of e, a power of two within 2^8 of d, so that f is exact there, and so are the mins: each half's
 // 8 go out with the half, minus the fp16 of dmin * m (rounded there as well) in two bf16 pieces (AM, AM +
-// 1024). e moves only when a block's d leaves that range; the rows' accumulators are rescaled only then
+// 1024; the first again at AM + 2048, 0 where it is not finite). e moves only when a block's d leaves that range; the rows' accumulators are rescaled only then
 // (RT, with a flag per row tile at RT + 128).
 template <>
 struct PfDec<kQ2_K> {
@@ -455,7 +455,7 @@ struct PfDec<kQ2_K> {
     const float re = pow2_inv(e);
     const uint32_t mine = (q < 2 ? w.sc.x : w.sc.y) >> (16 * (q & 1));  // groups 2q, 2q + 1: slice q's
     const float dmin = half_bits_to_float(w.dm >> 16);
-    uint32_t hi[2], lo[2];
+    uint32_t hi[2], lo[2], fin[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       c.mul[i] = h2_of(__half2float(__float2half_rn(d * (float)((mine >> (8 * i)) & 0xF))) * re);
@@ -463,9 +463,11 @@ struct PfDec<kQ2_K> {
       hi[i] = __float_as_uint(f) >> 16;  // the upper 8 bits of 11
       const float r = f - __uint_as_float(hi[i] << 16);
       lo[i] = __float_as_uint(r == r ? r : 0.0f) >> 16;
+      fin[i] = r == r ? hi[i] : 0;
     }
     *(uint32_t*)(s.AM + row * 8 + 2 * q) = hi[0] | (hi[1] << 16);
     *(uint32_t*)(s.AM + 1024 + row * 8 + 2 * q) = lo[0] | (lo[1] << 16);
+    *(uint32_t*)(s.AM + 2048 + row * 8 + 2 * q) = fin[0] | (fin[1] << 16);
     *(uint32_t*)(s.AM + 3072 + 1024 * (q >> 1) + row * 8 + 2 * q) = h2_bits(h2{c.mul[0][0], c.mul[1][0]});
     *(uint32_t*)(s.AM + 4096 - 1024 * (q >> 1) + row * 8 + 2 * q) = 0;
 #pragma unroll
