@@ -84,7 +84,11 @@ GGUF_API int gguf_check_op(int op, const gguf_view* W, const gguf_view* X, int64
                   const gguf_view* x_q8);
 
 /* Workspace bytes the op needs for n activation rows of K columns (the q8_1 copy of X unless
- * x_q8 is given). 0 if none. */
+ * x_q8 is given). 0 if none. Products of many rows run the fastest plan that fits the workspace
+ * they are given: with the bytes reported here the prefill GEMM in whole tiles or the small GEMM,
+ * by estimate; with room for partial sums after the copy (up to 64 MiB) the prefill GEMM with K
+ * split over the GPU, as gguf_mul_mat_alloc sizes it; with the int8 copy alone, half of what is
+ * reported, the small GEMM. */
 GGUF_API size_t gguf_op_workspace_bytes(int op, int64_t type, int64_t row, int64_t k, int64_t n, int has_x_q8);
 
 /* One product: Y[n, row] = X @ W[:row].T, written to y (y_bytes >= n*row*sizeof(X dtype)).
@@ -103,7 +107,8 @@ typedef void* (*gguf_alloc_fn)(void* ctx, int what, size_t bytes);
 /* gguf_mul_mat that takes its output and workspace from the caller's allocator once the guards
  * have passed: the order of the reference's run() (lcpp_shim.cu:767-805: the guards, then the
  * output from torch's allocator, then the launches), with one guard pass per call. The output is
- * asked for first, also when X has no rows; the workspace only when the plan needs one. */
+ * asked for first, also when X has no rows; the workspace only when the plan needs one (for the
+ * prefill GEMM the activation copy, up to 64 MiB of partial sums and a counter per tile). */
 GGUF_API int gguf_mul_mat_alloc(int op, const gguf_view* W, const gguf_view* X, int64_t type, int64_t row,
                                 const gguf_view* x_q8, gguf_alloc_fn alloc, void* alloc_ctx, void* stream);
 
@@ -115,9 +120,13 @@ GGUF_API size_t gguf_scratch_bytes(void);
  * reference; for callers that cannot allocate (code under stream capture, tight serving loops,
  * harnesses that forbid hipMalloc). The workspace is a statically sized device array of
  * GGUF_SCRATCH_BYTES per GPU, located once per device on the first call there and held until the
- * process ends. A product whose workspace (gguf_op_workspace_bytes) exceeds it is rejected with
- * GGUF_EINVAL; that covers the decode and small-batch products (e.g. 64 activation rows at
- * K = 17408) but not large prefills. Every call on a GPU shares that GPU's array: calls that
+ * process ends. It covers the decode and small-batch products (e.g. 64 activation rows at K =
+ * 17408) and prompts of moderate length. A product whose workspace (gguf_op_workspace_bytes)
+ * exceeds it is rejected with GGUF_EINVAL, but for those whose int8 activation copy fits it (4.5
+ * KiB per 16 rows and 256 columns): they run on that copy, or in parts of the activation rows.
+ * (IQ3_S and Q4_K with K <= 8192 have no plan on an int8 copy from 64 rows on; IQ3_S, Q4_K and
+ * Q6_K products of 256 rows or more on 64 tiles of 128 x 256 or more are rejected with their fp16
+ * copy, IQ3_XXS ones on 32, and from 64 rows on 128.) Every call on a GPU shares that GPU's array: calls that
  * overlap on one GPU (other streams, other threads) race, so the caller serialises them; the
  * scratch needs no clearing (every byte a kernel reads is written first by the same call). */
 GGUF_API int gguf_mul_mat_noalloc(int op, const gguf_view* W, const gguf_view* X, int64_t type, int64_t row,

@@ -201,3 +201,73 @@ def test_q2k_min_beyond_fp16(n, group):
     assert (sums > 0).any() and (sums < 0).any()
     assert np.array_equal(y[:, bad], np.repeat(want[:, None], len(bad), 1), equal_nan=True)
     assert np.isfinite(np.delete(y, bad, axis=1)).all()
+
+
+def _run_ws(lib, qt, w, x, rows, nbytes):
+    """gguf_mul_mat with a workspace of nbytes bytes: (rc, output, bytes of the workspace that were written,
+    counted to the last one; its fill is 0xFF)."""
+    from vllm_gguf_plugin import _capi
+
+    op, n = (PACKED_TILED if qt in PACKED else MUL_MAT_Q), x.shape[0]
+    y = torch.full((n, rows), float("nan"), dtype=x.dtype, device="cuda")
+    ws = torch.full((nbytes + 256,), 0xFF, dtype=torch.uint8, device="cuda")
+    rc = lib.gguf_mul_mat(op, _capi.ref(_capi.view(w)), _capi.ref(_capi.view(x)), qt, rows, None, y.data_ptr(),
+                          y.numel() * y.element_size(), ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    written = (ws != 0xFF).nonzero()
+    return rc, y, int(written[-1]) + 1 if len(written) else 0
+
+
+def _xh(qt, k, n):
+    return -(-n // 16) * (k // 256) * (8192 + (2560 if qt == o.Q2_K else 1024))
+
+
+def _int8(qt, k, n):
+    return n * k // 128 * 144 if qt == o.Q2_K else -(-n // 16) * (k // 256) * 4608
+
+
+# whole tiles of 128 rows on few CUs lose to the small GEMMs' 16-row tiles
+@pytest.mark.parametrize("qt,rows,k,n,whole", [
+    (o.IQ4_XS, 5120, 6144, 65, False), (o.IQ4_XS, 17408, 5120, 65, True), (o.IQ4_XS, 5120, 17408, 100, False),
+    (o.Q6_K, 5120, 17408, 100, False), (o.Q6_K, 34816, 5120, 65, True), (o.IQ2_S, 1024, 5120, 300, False),
+    (o.IQ2_XXS, 17408, 5120, 65, True), (o.IQ3_XXS, 1024, 5120, 257, False), (o.IQ3_S, 5120, 17408, 100, False),
+    (o.Q2_K, 1024, 5120, 16, False), (o.Q2_K, 5120, 17408, 16, False), (o.Q2_K, 17408, 5120, 100, True)])
+def test_whole_tiles_where_they_are_the_faster_plan(lib, qt, rows, k, n, whole):
+    """Without room for the split's parts a product runs the prefill GEMM in whole tiles only where that is
+    the faster plan, which shows in what it writes of a workspace of the reported size: the fp16 copy, or
+    the int8 one of half the size (and what its own split needs)."""
+    op = PACKED_TILED if qt in PACKED else MUL_MAT_Q
+    need = lib.gguf_op_workspace_bytes(op, qt, rows, k, n, 0)
+    assert need == _xh(qt, k, n)
+    w = torch.zeros(rows, o.BLOCK_BYTES[qt] * (k // 256), dtype=torch.uint8, device="cuda")
+    x = torch.randn(n, k, device="cuda")
+    rc, y, used = _run_ws(lib, qt, w, x, rows, need)
+    assert rc == 0 and (y == 0).all()
+    assert used > 0.9 * need if whole else used <= _int8(qt, k, n)
+    # a workspace with room for the int8 copy alone runs the small GEMM
+    rc, y, used = _run_ws(lib, qt, w, x, rows, -(-_int8(qt, k, n) // 256) * 256)
+    assert rc == 0 and (y == 0).all() and used <= _int8(qt, k, n)
+    rc, _, used = _run_ws(lib, qt, w, x, rows, _int8(qt, k, n) // 2)
+    assert rc != 0 and used == 0
+
+
+@pytest.mark.parametrize("qt,rows,k,n,taken", [
+    (o.IQ4_XS, 400, 5120, 1456, True), (o.IQ4_XS, 400, 5120, 1472, False), (o.IQ4_XS, 17408, 17408, 416, True),
+    (o.IQ3_S, 1024, 5120, 720, True), (o.IQ3_S, 1024, 5120, 1100, False), (o.Q4_K, 400, 5120, 1100, False),
+    (o.IQ3_S, 2048, 17408, 300, True), (o.IQ3_S, 8192, 17408, 300, False), (o.Q6_K, 400, 5120, 1400, True),
+    (o.Q6_K, 8192, 5120, 1400, False), (o.IQ3_XXS, 400, 5120, 1400, True), (o.IQ3_XXS, 4096, 5120, 1400, False),
+    (o.IQ2_XS, 17408, 5120, 1400, True), (o.Q2_K, 1024, 5120, 1456, True), (o.Q2_K, 1024, 5120, 1472, False)])
+def test_noalloc_takes_what_the_small_gemms_copy_fits(lib, qt, rows, k, n, taken):
+    """Beyond the scratch with its fp16 copy: taken where the small GEMM's workspace fits, refused on large
+    grids of the types whose prefill GEMM has always read the fp16 copy, and where nothing fits."""
+    from vllm_gguf_plugin import _capi
+
+    w = torch.zeros(rows, o.BLOCK_BYTES[qt] * (k // 256), dtype=torch.uint8, device="cuda")
+    x = torch.randn(n, k, device="cuda", dtype=torch.bfloat16)
+    y = torch.full((n, rows), float("nan"), dtype=x.dtype, device="cuda")
+    rc = lib.gguf_mul_mat_noalloc(PACKED_TILED if qt in PACKED else MUL_MAT_Q, _capi.ref(_capi.view(w)),
+                                  _capi.ref(_capi.view(x)), qt, rows, None, y.data_ptr(), y.numel() * 2,
+                                  torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert (rc == 0) == taken, _capi.error(lib)
+    assert (y == 0).all() if taken else "static scratch" in _capi.error(lib)

@@ -8,7 +8,9 @@
 // Q4_K, Q6_K, IQ2_XXS, IQ2_XS, IQ2_S, IQ3_XXS, IQ3_S, IQ4_XS, IQ1_M; lcpp_shim.cu:676-684).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <mutex>
@@ -62,8 +64,10 @@ bool small_h_supported(int type, bool packed);
 bool small_h_range(int type, int64_t nrows, int64_t n);
 hipError_t launch_gemm_small_h(int type, bool packed, const uint8_t* W, int64_t row_bytes, int nrows, int k,
                                const uint8_t* xh, int n, void* y, int y_dtype, hipStream_t stream);
-hipError_t launch_gemm_prefill(int type, bool exact, const uint8_t* W, int64_t row_bytes, int nrows, int k, const uint8_t* xh, int n,
-                               void* y, int y_dtype, float* part, uint32_t* cnt, hipStream_t stream);
+double prefill_whole_us(int type, bool exact, int64_t nrows, int64_t k, int64_t n);
+hipError_t launch_gemm_prefill(int type, bool exact, bool split, const uint8_t* W, int64_t row_bytes, int nrows, int k,
+                               const uint8_t* xh, int n, void* y, int y_dtype, float* part, uint32_t* cnt,
+                               hipStream_t stream);
 hipError_t launch_iq3_pack(int type, uint8_t* w, int64_t rows, int64_t row_bytes, bool unpack, uint8_t* scratch,
                            size_t scratch_bytes, hipStream_t stream);
 size_t iq3_pack_scratch_bytes(int64_t rows, int64_t row_bytes);
@@ -266,10 +270,10 @@ bool xxs_packed(int op, int64_t type);
 
 bool small_fp16_shape(int op, int64_t type, int64_t k, int64_t n);
 
-// Whether a product op runs the prefill GEMM (gemm_prefill.hip): a tile of 128 weight rows decoded
-// once per step for up to 256 columns, work split evenly over the CUs, against the small GEMMs'
-// 16-row tiles that decode the weights again for every 4 column tiles. Measured (us per op, graph
-// replays, prefill / the plan it replaces):
+// Whether a product op runs the prefill GEMM (gemm_prefill.hip) where its workspace has room for the split
+// plan: a tile of 128 weight rows decoded once per step for up to 256 columns, work split evenly over the
+// CUs, against the small GEMMs' 16-row tiles that decode the weights again for every 4 column tiles.
+// Measured (us per op, graph replays, prefill / the plan it replaces):
 //   34816 x 5120, M = 65 / 256 / 512: IQ3_S 83 / 145 / 257 against 149 / 234 / 353, IQ4_XS 98 / 175 /
 //   317 against 251 / 393 / 607, Q6_K 94 / 151 / 270 against 322 / 249 / 376, IQ2_S 85 / 134 / 254
 //   against 310 / 640 / 1264; 5120 x 6144, M = 65: IQ3_S 31 against 45, Q6_K 32 against 68.
@@ -292,6 +296,40 @@ bool prefill_route(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
 // GEMM's are: two MFMAs per slice instead of one.
 bool q6k_rounded(int64_t type, int64_t row, int64_t n) {
   return type == gguf::kQ6_K && n >= 256 && (row + 127) / 128 * ((n + 255) / 256) >= 64;
+}
+
+// Estimated time of the small GEMM that a product runs without the prefill GEMM, us: K blocks x workgroups
+// (a 16-row tile and up to four column tiles) per CU x a block's time in one. Q2_K's per-slice GEMM: a
+// workgroup alone on its CU takes 1.6 times that. Fitted like pf_whole_shape's.
+double small_us(int64_t type, int64_t row, int64_t k, int64_t n) {
+  const int64_t nct = (n + 15) / 16, nb = k / 256;
+  const double tiles = (double)((row + 15) / 16) / 256;
+  if (type == gguf::kQ2_K) {
+    const double wgs = std::ceil(tiles * std::max(1.0, (double)nct / 4));
+    return 12 + (double)nb * (0.35 + 0.33 * (double)std::min<int64_t>(nct, 4)) * std::max(1.6, wgs);
+  }
+  const bool deep = k > 8192;  // IQ3_S and Q4_K run the int8 GEMM instead of the fp16 one
+  double per = deep ? 0.78 : 0.76;  // IQ3_XXS, IQ2_S, IQ2_XS
+  if (type == gguf::kIQ2_XXS) per = deep ? 0.66 : 0.76;
+  if (type == gguf::kIQ3_S) per = deep ? 0.76 : 0.42;
+  if (type == gguf::kQ4_K) per = deep ? 0.52 : 0.50;
+  if (type == gguf::kQ6_K) per = deep ? 0.64 : 0.94;
+  if (type == gguf::kIQ4_XS) per = deep ? 0.56 : 0.60;
+  return 12 + (double)nb * per * tiles * (double)((nct + 3) / 4);
+}
+
+// Whether a product of prefill_route runs the prefill GEMM without room for the split plan's parts, in
+// whole tiles: a tile walks all of K, so on a grid of few tiles most CUs idle, and the small GEMMs, whose
+// 16-row tiles spread the same work, are the faster ones. By the estimates of both. Measured, us, whole
+// tiles (their best width) / small GEMM / split plan: 5120 x 17408 M = 100 IQ3_S 140 / 132 / 63, Q2_K 226 /
+// 323 / 78, M = 512 IQ3_S 200 / 432 / 145; 5120 x 6144 M = 65 IQ3_S 56 / 38 / 33, Q6_K 80 / 68 / 38; 1024 x
+// 5120 M = 512 IQ3_S 52 / 31 / 30; 34816 x 5120 M = 65 IQ3_S 121 / 117 / 85, IQ2_S 121 / 299 / 82. Over 12
+// shapes and 14 row counts of each type the choice is within 1 % of the better one on average, at worst
+// 18 % (IQ3_S 34816 x 5120 M = 160 194 against 164), and at worst 4 % slower than the GEMM that ran before
+// the split plan took the product over.
+bool whole_route(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
+  return prefill_route(op, type, row, k, n) &&
+         gguf::prefill_whole_us((int)type, !q6k_rounded(type, row, n), row, k, n) < small_us(type, row, k, n);
 }
 
 // Where the prefill GEMM is the faster one below those rows, but its activation copy is twice the
@@ -356,7 +394,7 @@ bool rows_fused(int op, int64_t type, int64_t row, int64_t k, int64_t n, bool ha
   return bb > 0 && gguf::gemv_rows_x_supported((int)type, row, k / 256 * bb, k, n);
 }
 
-// The MFMA products with K <= 8192 below the prefill GEMM's rows run the fp16 small GEMM (X in the xh
+// The MFMA products with K <= 8192 off the prefill GEMM run the fp16 small GEMM (X in the xh
 // layout) for packed IQ3_S and Q4_K from 64 activation rows, and below 64 where its
 // one-workgroup-per-CU range plan applies (4..5 row tiles per CU; 33..48 rows for IQ3_S, 17..48 for
 // Q4_K); the rest the int8 small GEMM (xq layout).
@@ -365,21 +403,21 @@ bool small_fp16_shape(int op, int64_t type, int64_t k, int64_t n) {
 }
 bool small_fp16(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
   if (!small_fp16_shape(op, type, k, n)) return false;
-  return (n >= 64 && !prefill_route(op, type, row, k, n)) || gguf::small_h_range((int)type, row, n);
+  return n >= 64 || gguf::small_h_range((int)type, row, n);
 }
 
-// The int8 small GEMM on Q4_K / IQ4_XS / Q6_K rows (gemm_raw_kernel): product ops below the
-// prefill rows off the fp16 GEMM's plans, and decode ops from vec_mma_from rows on.
+// The int8 small GEMM on Q4_K / IQ4_XS / Q6_K rows (gemm_raw_kernel): product ops off the prefill
+// and the fp16 GEMM's plans, and decode ops from vec_mma_from rows on.
 bool raw_gemm(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
   if (op_packed(op) || !(type == gguf::kQ4_K || type == gguf::kIQ4_XS || type == gguf::kQ6_K)) return false;
-  if (op_gemm(op)) return !prefill_route(op, type, row, k, n) && !small_fp16(op, type, row, k, n);
+  if (op_gemm(op)) return !small_fp16(op, type, row, k, n);
   return decode_mma(op, type, row, k, n);
 }
 
 // The int8 tile GEMM on packed IQ3_S (gemm_iq3s_tile_kernel), on the same terms.
 bool tile_gemm(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
   if (!op_packed(op) || type != gguf::kIQ3_S) return false;
-  if (op_gemm(op)) return !prefill_route(op, type, row, k, n) && !small_fp16(op, type, row, k, n);
+  if (op_gemm(op)) return !small_fp16(op, type, row, k, n);
   return decode_mma(op, type, row, k, n);
 }
 
@@ -396,26 +434,23 @@ SplitPlan split_plan(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
   return p;
 }
 
-// Bytes of a prefill product's workspace with its split plan: the xh copy of X, the partial sums and
-// the tile counters. gguf_op_workspace_bytes reports the copy alone: with no more than that the
-// product runs unsplit.
-size_t prefill_split_ws(int64_t type, int64_t row, int64_t k, int64_t n) {
-  const size_t slots = gguf::prefill_slot_bytes(row, k, n);
-  const size_t xh = align256(gguf::xh_bytes(n, k, (int)type));
-  return slots ? xh + slots + align256((size_t)gguf::prefill_counters(row, k, n) * 4) : xh;
-}
-
 // Bytes after the xq copy of X that a split GEMM needs (slots, then its counters).
 size_t split_ws(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
   const SplitPlan p = split_plan(op, type, row, k, n);
   return gguf::split_ws_bytes(p.split, p.tiles, n);
 }
 
-}  // namespace
+// Bytes of the activation copy of a prefill product, and with its split plan: the copy, the partial sums and
+// the tile counters.
+size_t prefill_ws(int64_t type, int64_t k, int64_t n) { return align256(gguf::xh_bytes(n, k, (int)type)); }
+size_t prefill_split_ws(int64_t type, int64_t row, int64_t k, int64_t n) {
+  const size_t slots = gguf::prefill_slot_bytes(row, k, n);
+  const size_t cnt = slots ? align256((size_t)gguf::prefill_counters(row, k, n) * 4) : 0;
+  return prefill_ws(type, k, n) + slots + cnt;
+}
 
-size_t gguf_op_workspace_bytes(int op, int64_t type, int64_t row, int64_t k, int64_t n, int has_x_q8) {
-  if (n <= 0) return 0;
-  if (prefill_route(op, type, row, k, n)) return align256(gguf::xh_bytes(n, k, (int)type));
+// Workspace bytes of an op off the prefill GEMM.
+size_t small_ws(int op, int64_t type, int64_t row, int64_t k, int64_t n, bool has_x_q8) {
   if (generic(type)) {
     if (op_gemm(op)) return align256(generic_xq(type) ? gguf::xq_bytes(n, k) : gguf_q8_1_bytes(n, k, 1));
     return has_x_q8 || generic_fused(op, type, row, k, n) ? 0 : align256(gguf_q8_1_bytes(n, k, 0));
@@ -427,8 +462,28 @@ size_t gguf_op_workspace_bytes(int op, int64_t type, int64_t row, int64_t k, int
   }
   if (decode_mma(op, type, row, k, n))  // x_q8 is converted into it
     return align256(gguf::xq_bytes(n, k)) + split_ws(op, type, row, k, n);
-  if (packed_fused(op, row, k, n, has_x_q8 != 0) || rows_fused(op, type, row, k, n, has_x_q8 != 0)) return 0;
+  if (packed_fused(op, row, k, n, has_x_q8) || rows_fused(op, type, row, k, n, has_x_q8)) return 0;
   return has_x_q8 ? 0 : align256(gguf_q8_1_bytes(n, k, 0));
+}
+
+// How an op runs: off the prefill GEMM, or on it in whole tiles or with K split over the CUs.
+enum class Plan { kSmall, kWhole, kSplit };
+
+// The plan of a workspace of `bytes` bytes: the fastest one that fits it (kSmall, which may not fit either,
+// if none does).
+Plan plan_for(int op, int64_t type, int64_t row, int64_t k, int64_t n, size_t bytes) {
+  if (!prefill_route(op, type, row, k, n) || bytes < prefill_ws(type, k, n)) return Plan::kSmall;
+  if (bytes >= prefill_split_ws(type, row, k, n)) return Plan::kSplit;
+  return whole_route(op, type, row, k, n) ? Plan::kWhole : Plan::kSmall;
+}
+
+}  // namespace
+
+// The larger of the prefill GEMM's activation copy and the small GEMM's workspace where either may run.
+size_t gguf_op_workspace_bytes(int op, int64_t type, int64_t row, int64_t k, int64_t n, int has_x_q8) {
+  if (n <= 0) return 0;
+  const size_t small = small_ws(op, type, row, k, n, has_x_q8 != 0);
+  return prefill_route(op, type, row, k, n) ? std::max(small, prefill_ws(type, k, n)) : small;
 }
 
 }  // extern "C"
@@ -436,12 +491,11 @@ size_t gguf_op_workspace_bytes(int op, int64_t type, int64_t row, int64_t k, int
 namespace {
 
 // One product whose guards have passed (check_op returned k): the buffer checks, the plan and the
-// launches. Every entry point runs the guards once and then this. prefill: the prefill GEMM runs it
-// (prefill_route or prefill_preferred); its tiles' K is split where the workspace has room for the
-// parts.
+// launches. Every entry point runs the guards once and then this. fixed_plan: how it runs, or null: as the
+// workspace allows (plan_for, asked on X's device).
 int run_checked(int op, const gguf_view* W, const gguf_view* X, int64_t type, int64_t row, const gguf_view* x_q8,
                 int64_t k, void* y, size_t y_bytes, void* workspace, size_t workspace_bytes, void* stream,
-                bool prefill) {
+                const Plan* fixed_plan = nullptr) {
   const char* name = op_name(op);
   const int64_t n = X->size[0];
   if (n == 0) return GGUF_OK;
@@ -452,8 +506,10 @@ int run_checked(int op, const gguf_view* W, const gguf_view* X, int64_t type, in
   const DeviceScope scope(X->device);
   if (scope.err != hipSuccess) return hip_fail(scope.err, name, "device select");
   // sized on X's device, as the dispatch below decides (some plans depend on its CU count)
-  const size_t need = prefill ? align256(gguf::xh_bytes(n, k, (int)type))
-                              : gguf_op_workspace_bytes(op, type, row, k, n, x_q8 != nullptr);
+  const Plan plan = fixed_plan ? *fixed_plan : plan_for(op, type, row, k, n, workspace_bytes);
+  const size_t need = plan == Plan::kSplit   ? prefill_split_ws(type, row, k, n)
+                      : plan == Plan::kWhole ? prefill_ws(type, k, n)
+                                             : small_ws(op, type, row, k, n, x_q8 != nullptr);
   if (workspace_bytes < need || (need > 0 && !workspace))
     return fail("%s: workspace of %zu bytes needed, got %zu", name, need, workspace_bytes);
   if (reinterpret_cast<uintptr_t>(workspace) % 16 != 0) return fail("%s: workspace must be 16-byte aligned", name);
@@ -463,19 +519,21 @@ int run_checked(int op, const gguf_view* W, const gguf_view* X, int64_t type, in
   const int64_t row_bytes = W->size[1];
   const int ydt = X->dtype;
 
-  if (prefill) {
+  if (plan != Plan::kSmall) {
     uint8_t* ws = (uint8_t*)workspace;
     float* part = nullptr;
     uint32_t* cnt = nullptr;
-    const size_t slots = gguf::prefill_slot_bytes(row, k, n);
-    if (slots && workspace_bytes >= prefill_split_ws(type, row, k, n)) {
-      part = (float*)(ws + align256(gguf::xh_bytes(n, k, (int)type)));
+    const bool split = plan == Plan::kSplit;
+    const size_t slots = split ? gguf::prefill_slot_bytes(row, k, n) : 0;
+    if (slots) {
+      part = (float*)(ws + prefill_ws(type, k, n));
       cnt = (uint32_t*)((uint8_t*)part + slots);
     }
     e = gguf::launch_quantize_xh(X->data, X->dtype, n, k, s01, (int)type, ws, s, cnt,
                                  cnt ? gguf::prefill_counters(row, k, n) : 0);
     if (e != hipSuccess) return hip_fail(e, name, "quantize");
-    e = gguf::launch_gemm_prefill((int)type, !q6k_rounded(type, row, n), w, row_bytes, (int)row, (int)k, ws, (int)n, y, ydt, part, cnt, s);
+    e = gguf::launch_gemm_prefill((int)type, !q6k_rounded(type, row, n), split, w, row_bytes, (int)row, (int)k, ws, (int)n,
+                                  y, ydt, part, cnt, s);
     if (e != hipSuccess) return hip_fail(e, name, "gemm");
     return GGUF_OK;
   }
@@ -611,8 +669,7 @@ int gguf_mul_mat(int op, const gguf_view* W, const gguf_view* X, int64_t type, i
   g_err.clear();
   const int64_t k = check_op(op, W, X, type, row, x_q8);
   if (k < 0) return GGUF_EINVAL;
-  return run_checked(op, W, X, type, row, x_q8, k, y, y_bytes, workspace, workspace_bytes, stream,
-                     prefill_route(op, type, row, k, X->size[0]));
+  return run_checked(op, W, X, type, row, x_q8, k, y, y_bytes, workspace, workspace_bytes, stream);
 }
 
 int gguf_mul_mat_alloc(int op, const gguf_view* W, const gguf_view* X, int64_t type, int64_t row,
@@ -629,15 +686,15 @@ int gguf_mul_mat_alloc(int op, const gguf_view* W, const gguf_view* X, int64_t t
   if (n == 0) return GGUF_OK;
   const DeviceScope scope(X->device);
   if (scope.err != hipSuccess) return hip_fail(scope.err, name, "device select");
-  const bool prefill = prefill_preferred(op, type, row, k, n);
-  const size_t need = prefill ? prefill_split_ws(type, row, k, n)
-                              : gguf_op_workspace_bytes(op, type, row, k, n, x_q8 != nullptr);
+  const Plan plan = prefill_preferred(op, type, row, k, n) ? Plan::kSplit : Plan::kSmall;
+  const size_t need = plan == Plan::kSplit ? prefill_split_ws(type, row, k, n)
+                                           : small_ws(op, type, row, k, n, x_q8 != nullptr);
   void* ws = nullptr;
   if (need) {
     ws = alloc(alloc_ctx, GGUF_ALLOC_WORKSPACE, need);
     if (!ws) return fail("%s: the allocator returned no workspace", name);
   }
-  return run_checked(op, W, X, type, row, x_q8, k, y, y_bytes, ws, need, stream, prefill);
+  return run_checked(op, W, X, type, row, x_q8, k, y, y_bytes, ws, need, stream, &plan);
 }
 
 }  // extern "C"
@@ -650,17 +707,15 @@ namespace {
 // device current, once, and is kept here.
 __device__ __align__(256) uint8_t scratch[kScratchBytes];
 
-// Products of the prefill GEMM that this entry point takes although its fp16 activation copy exceeds
-// the scratch: those whose int8 copy (xq, 4.5 KB per 16 rows and K block; block_q8_1_mmq for Q2_K)
-// fits it, on weights and types that the fp16 layout's int8 predecessor served.
-bool noalloc_in_parts(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
-  if (type == gguf::kQ2_K) return align256(gguf_q8_1_bytes(n, k, 1)) <= kScratchBytes;
+// Whether the no-allocation entry point takes a product whose reported workspace exceeds the scratch: where
+// the small GEMM's fits it. Products on large grids of the types whose prefill GEMM has always read the
+// fp16 copy are refused with it, as they always were.
+bool noalloc_beyond_scratch(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
   const int64_t groups = (row + 127) / 128 * ((n + 255) / 256);
-  const bool fp16 = xxs_packed(op, type) ? (n >= 256 && groups >= 32) || groups >= 128
-                    : (type == gguf::kIQ3_S || type == gguf::kQ4_K || type == gguf::kQ6_K)
-                        ? (n >= 256 && groups >= 64) || (n < 256 && small_fp16_shape(op, type, k, n))
-                        : false;
-  return !fp16 && align256(gguf::xq_bytes(n, k)) + split_ws(op, type, row, k, n) <= kScratchBytes;
+  const bool fp16 = xxs_packed(op, type) ? (n >= 256 && groups >= 32) || (n >= 64 && groups >= 128)
+                    : type == gguf::kIQ3_S || type == gguf::kQ4_K || type == gguf::kQ6_K ? n >= 256 && groups >= 64
+                                                                                         : false;
+  return prefill_route(op, type, row, k, n) && !fp16 && small_ws(op, type, row, k, n, false) <= kScratchBytes;
 }
 
 void* g_scratch_ptr[gguf::kMaxDevices] = {};
@@ -700,25 +755,34 @@ int gguf_mul_mat_noalloc(int op, const gguf_view* W, const gguf_view* X, int64_t
   const DeviceScope scope(X->device);
   if (scope.err != hipSuccess) return hip_fail(scope.err, name, "device select");
   const size_t need = gguf_op_workspace_bytes(op, type, row, k, n, x_q8 != nullptr);
-  const bool prefill = prefill_route(op, type, row, k, n);
-  if (need > kScratchBytes && !(prefill && noalloc_in_parts(op, type, row, k, n)))
+  if (need > kScratchBytes && !noalloc_beyond_scratch(op, type, row, k, n))
     return fail("%s: needs a %zu-byte workspace, more than the %zu-byte static scratch of the no-allocation "
                 "entry point (use gguf_mul_mat with a workspace)", name, need, kScratchBytes);
   if (y_bytes < (size_t)(n * row * elem_size(X->dtype))) return fail("%s: output buffer too small", name);
   void* ws = nullptr;
   const hipError_t e = scratch_address(X->device, &ws);
   if (e != hipSuccess) return hip_fail(e, name, "scratch address");
-  if (need <= kScratchBytes) return run_checked(op, W, X, type, row, x_q8, k, y, y_bytes, ws, need, stream, prefill);
-  // activation rows in parts whose copy fits the scratch, one after the other on the stream
+  // the reported size, not the scratch's: the same plan and so the same bits as with a workspace of that size
+  if (need <= kScratchBytes) return run_checked(op, W, X, type, row, x_q8, k, y, y_bytes, ws, need, stream);
+  // whole tiles over activation rows in parts whose copy fits the scratch, one after the other on the
+  // stream, where that is estimated the faster one; else the small GEMM
   const int64_t es = elem_size(X->dtype);
   int64_t part = (int64_t)(kScratchBytes / gguf::xh_bytes(16, k, (int)type)) * 16;
   if (part >= 256) part -= part % 256;  // whole column groups
+  Plan plan = Plan::kSmall;
+  if (part > 0) {
+    const bool exact = !q6k_rounded(type, row, n);
+    const double us = (double)(n / part) * gguf::prefill_whole_us((int)type, exact, row, k, part) +
+                      (n % part ? gguf::prefill_whole_us((int)type, exact, row, k, n % part) : 0);
+    if (us < small_us(type, row, k, n)) plan = Plan::kWhole;
+  }
+  if (plan == Plan::kSmall) part = n;
   for (int64_t c = 0; c < n; c += part) {
     gguf_view xp = *X;
     xp.data = (const uint8_t*)X->data + c * X->stride[0] * es;
     xp.size[0] = n - c < part ? n - c : part;
     const int rc = run_checked(op, W, &xp, type, row, x_q8, k, (uint8_t*)y + c * row * es, y_bytes - c * row * es, ws,
-                               kScratchBytes, stream, true);
+                               kScratchBytes, stream, &plan);
     if (rc != GGUF_OK) return rc;
   }
   return GGUF_OK;

@@ -491,7 +491,9 @@ struct PfShape {
 // IQ3_S, K = 5120, slopes and intercepts over rows and K splits: block 3.5 / 2.3 / 1.7 us with a few
 // workgroups and 5.6 / 3.0 / 2.3 with 256 for rs = 1 / 2 / 4, fixed 20 / 16 / 14. Measured at rs =
 // 1 / 2 / 4: 1024 rows M = 256 48 / 32 / 25 us, 8192 rows M = 128 49 / 33 / 34, 34816 rows M = 100
-// 133 / 89 / 115, M = 512 271 / 305 / 400.
+// 133 / 89 / 115, M = 512 271 / 305 / 400. For the other types it takes the fastest rs as well, within 1 %
+// on average over 12 shapes and 14 row counts each, at worst 19 % (6144 x 2048 M = 300 IQ4_XS, 40 us at rs = 2
+// against 33 at 4).
 PfShape pf_shape(int64_t nrows, int64_t k, int64_t n) {
   static const double fixed[3] = {20, 16, 14}, few[3] = {3.5, 2.3, 1.7}, full[3] = {5.6, 3.0, 2.3};
   const int64_t nct = xq_col_tiles(n), nb = k / kQK, nrg = (nrows + 127) / 128, cus = device_cus();
@@ -507,11 +509,29 @@ PfShape pf_shape(int64_t nrows, int64_t k, int64_t n) {
   return best;
 }
 
+// Whole tiles, where there is no room for parts: the rounds of tiles over the CUs, each whole[rs] + K
+// blocks x block[cost class][rs] us, least squares over 12 shapes (1024 x 5120 .. 34816 x 5120, K 2048 ..
+// 17408) and 65 .. 2048 rows, errors within -24 .. +14 % where one round fills few CUs, 10 % elsewhere.
+// Measured at rs = 1 / 2 / 4: IQ3_S 5120 x 6144 M = 128 112 / 77 / 58 us, M = 1024 125 / 162 / 167; 34816 x
+// 5120 M = 512 299 / 314 / 408.
+PfShape pf_whole_shape(int type, bool exact, int64_t nrows, int64_t k, int64_t n, double* us) {
+  static const double whole[3] = {14, 11, 8.5}, block[3][3] = {{4.1, 2.75, 2.0}, {5.5, 3.3, 2.2}, {6.2, 4.2, 3.2}};
+  const int cost = type == kIQ4_XS ? 1 : type == kQ2_K || (type == kQ6_K && exact) ? 2 : 0;
+  const int64_t nct = xq_col_tiles(n), nb = k / kQK, nrg = (nrows + 127) / 128, cus = device_cus();
+  PfShape best{1, 0, 0};
+  for (int i = 0; i < 3; ++i) {
+    const int64_t per = 16 >> i, tiles = nrg * ((nct + per - 1) / per);
+    const double t = (double)((tiles + cus - 1) / cus) * (whole[i] + (double)nb * block[cost][i]);
+    if (i == 0 || t < *us) *us = t, best = {1 << i, tiles, std::min(cus, tiles)};
+  }
+  return best;
+}
+
 template <int TYPE, int RS>
 void launch_prefill_h(const PfShape& s, const uint8_t* W, int64_t row_bytes, int nrows, int k, const uint8_t* xh, int n,
                       void* y, int y_dtype, float* part, uint32_t* cnt, hipStream_t stream) {
   const int64_t nb = k / kQK, tiles = s.tiles;
-  const bool split = part != nullptr;
+  const bool split = part != nullptr;  // else runs of whole tiles
   PfPlan p;
   p.ub = split ? 1 : (int)nb;
   p.nrg = (nrows + 127) / 128;
@@ -525,9 +545,8 @@ void launch_prefill_h(const PfShape& s, const uint8_t* W, int64_t row_bytes, int
 }
 
 template <int TYPE>
-void launch_prefill_t(const uint8_t* W, int64_t row_bytes, int nrows, int k, const uint8_t* xh, int n, void* y,
-                      int y_dtype, float* part, uint32_t* cnt, hipStream_t stream) {
-  const PfShape s = pf_shape(nrows, k, n);
+void launch_prefill_t(const PfShape& s, const uint8_t* W, int64_t row_bytes, int nrows, int k, const uint8_t* xh, int n,
+                      void* y, int y_dtype, float* part, uint32_t* cnt, hipStream_t stream) {
   switch (s.rs) {
     case 1: launch_prefill_h<TYPE, 1>(s, W, row_bytes, nrows, k, xh, n, y, y_dtype, part, cnt, stream); break;
     case 2: launch_prefill_h<TYPE, 2>(s, W, row_bytes, nrows, k, xh, n, y, y_dtype, part, cnt, stream); break;
@@ -555,13 +574,24 @@ size_t prefill_slot_bytes(int64_t nrows, int64_t k, int64_t n) {
   return (size_t)(s.wgs + std::min(s.wgs, s.tiles)) * (16 / s.rs) * 2 * 4096;
 }
 
-// Large-M products; xh: X in the xh layout of the type; part: prefill_slot_bytes of workspace, with
-// prefill_counters counters that the quantise launch cleared at cnt, or null: no tile is split. exact: Q6_K's
-// operands without the rounding beyond 2048 (two MFMAs per slice).
-hipError_t launch_gemm_prefill(int type, bool exact, const uint8_t* W, int64_t row_bytes, int nrows, int k, const uint8_t* xh, int n,
-                               void* y, int y_dtype, float* part, uint32_t* cnt, hipStream_t stream) {
+// Estimated time of a product in whole tiles, us.
+double prefill_whole_us(int type, bool exact, int64_t nrows, int64_t k, int64_t n) {
+  double us = 0;
+  pf_whole_shape(type, exact, nrows, k, n, &us);
+  return us;
+}
+
+// Large-M products; xh: X in the xh layout of the type. split: K over the CUs, with prefill_slot_bytes of
+// workspace at part and prefill_counters counters that the quantise launch cleared at cnt (both null where
+// the split needs no slots); else whole tiles. exact: Q6_K's operands without the rounding beyond 2048 (two
+// MFMAs per slice).
+hipError_t launch_gemm_prefill(int type, bool exact, bool split, const uint8_t* W, int64_t row_bytes, int nrows, int k,
+                               const uint8_t* xh, int n, void* y, int y_dtype, float* part, uint32_t* cnt,
+                               hipStream_t stream) {
+  double us = 0;
+  const PfShape s = split ? pf_shape(nrows, k, n) : pf_whole_shape(type, exact, nrows, k, n, &us);
 #define GGUF_PF(T) \
-  case T: launch_prefill_t<T>(W, row_bytes, nrows, k, xh, n, y, y_dtype, part, cnt, stream); break;
+  case T: launch_prefill_t<T>(s, W, row_bytes, nrows, k, xh, n, y, y_dtype, part, cnt, stream); break;
   switch (type == kQ6_K && exact ? kQ6_KX : type) {
     GGUF_PF(kQ6_KX)
     GGUF_PF(kIQ3_S)
