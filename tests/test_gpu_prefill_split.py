@@ -80,7 +80,8 @@ def test_split_and_unsplit_exact(lib, qt, rows, k, n):
 
 @pytest.mark.parametrize("n", [1, 8, 16, 17, 63, 64, 65, 128, 129])
 def test_q2k_every_row_count(n):
-    """Q2_K's product op runs the prefill GEMM at any row count: 64-column tiles (four row parts)."""
+    """Q2_K's product op at every row count: the prefill GEMM from 17 rows at this K (64-column tiles, four
+    row parts), the per-slice GEMM below; one row on the prefill GEMM: test_q2k_scales_rounded_as_the_model."""
     raw = exact_weights(o.Q2_K, 270, 2560, seed=n)
     x = exact_x(n, 2560, seed=n + 1, dtype=torch.float32)
     y = _torch_op(o.Q2_K, dev(raw), x.cuda(), 270).cpu().numpy()
@@ -155,8 +156,9 @@ def test_q2k_group_sum_beyond_fp16(n):
     assert np.isfinite(np.delete(y, 1, axis=0)).all()
 
 
-# (270, 2560, 24) and (270, 2560, 300): 64-column tiles; (4102, 2560, 600): 128; (16390, 2560, 1000): 256
-@pytest.mark.parametrize("rows,k,n", [(270, 2560, 24), (270, 2560, 300), (4102, 2560, 600), (16390, 2560, 1000)])
+# 64-column tiles; (4102, 2560, 600): 128; (16390, 2560, 1000): 256
+@pytest.mark.parametrize("rows,k,n", [(270, 5120, 1), (270, 5120, 8), (270, 2560, 24), (270, 2560, 300),
+                                      (4102, 2560, 600), (16390, 2560, 1000)])
 @pytest.mark.parametrize("scales", ["ordinary", "subnormal", "wide"])
 def test_q2k_scales_rounded_as_the_model(rows, k, n, scales):
     """Q2_K's products keep d times sub-scale as fp16, as the reference's tile loader does: fp32 X against
@@ -184,7 +186,7 @@ def test_q2k_min_beyond_fp16(n, group):
     """A min that overflows fp16 (dmin * m as the tile loader keeps it) of a group whose sum is stored
     (0..5 of each 128 values) or taken from q8 (6, 7): the weight row's outputs are minus the sum's
     infinity; the other rows stay finite."""
-    rows, k = 144, 1024
+    rows, k = 144, 5120
     raw = w_rand(o.Q2_K, rows, k, seed=9)
     blk = raw.reshape(rows, k // 256, 84)
     bad = np.arange(0, rows, 7)
@@ -271,3 +273,58 @@ def test_noalloc_takes_what_the_small_gemms_copy_fits(lib, qt, rows, k, n, taken
     torch.cuda.synchronize()
     assert (rc == 0) == taken, _capi.error(lib)
     assert (y == 0).all() if taken else "static scratch" in _capi.error(lib)
+
+
+def _asked(lib, qt, w, x, rows):
+    """gguf_mul_mat_alloc: (output, bytes of the workspace it asked for)."""
+    from vllm_gguf_plugin import _capi
+
+    n, got = x.shape[0], {}
+
+    def alloc(_, what, nbytes):
+        got[what] = torch.full((max(nbytes, 1),), 0xFF, dtype=torch.uint8, device="cuda")
+        got[what, "bytes"] = nbytes
+        return got[what].data_ptr()
+
+    fn = _capi.ALLOC_FN(alloc)
+    rc = lib.gguf_mul_mat_alloc(PACKED_TILED if qt in PACKED else MUL_MAT_Q, _capi.ref(_capi.view(w)),
+                                _capi.ref(_capi.view(x)), qt, rows, None, fn, None,
+                                torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, _capi.error(lib)
+    torch.cuda.synchronize()
+    y = got[_capi.ALLOC_OUTPUT][:n * rows * x.element_size()].view(x.dtype).view(n, rows)
+    return y, got[_capi.ALLOC_WORKSPACE, "bytes"]
+
+
+# small products, few rows of a deep K, and few activation rows are faster on the small GEMMs
+@pytest.mark.parametrize("qt,rows,k,n,split", [
+    (o.IQ4_XS, 512, 512, 300, False), (o.IQ4_XS, 1024, 1024, 300, False), (o.IQ4_XS, 1024, 512, 1024, True),
+    (o.IQ2_S, 512, 512, 300, False), (o.IQ2_S, 1024, 2048, 257, True), (o.Q6_K, 1024, 1024, 512, False),
+    (o.IQ4_XS, 1024, 17408, 100, False), (o.IQ4_XS, 1024, 17408, 129, True), (o.Q6_K, 512, 17408, 512, False),
+    (o.Q4_K, 2048, 17408, 65, False), (o.Q4_K, 3072, 17408, 65, True), (o.IQ2_XS, 1024, 17408, 65, True),
+    (o.IQ3_XXS, 8192, 5120, 33, False), (o.IQ3_XXS, 17408, 5120, 33, True), (o.IQ3_XXS, 4096, 4096, 64, True),
+    (o.IQ4_XS, 2048, 17408, 49, False), (o.IQ4_XS, 3072, 17408, 33, False), (o.IQ4_XS, 3072, 17408, 49, True),
+    (o.Q2_K, 1024, 1024, 16, False), (o.Q2_K, 1024, 2048, 32, False), (o.Q2_K, 1024, 2048, 48, True),
+    (o.Q2_K, 12288, 5120, 1, True)])
+def test_split_where_it_is_the_faster_plan(lib, qt, rows, k, n, split):
+    """The workspace the library sizes itself: with the split's parts (a slot of 2 x 4096 bytes for each row
+    tile and column pair of a workgroup's tile, a counter a tile) only where that plan is the faster one; the
+    small GEMM's otherwise, of at most the int8 copy and its own split."""
+    w = torch.zeros(rows, o.BLOCK_BYTES[qt] * (k // 256), dtype=torch.uint8, device="cuda")
+    y, asked = _asked(lib, qt, w, torch.randn(n, k, device="cuda"), rows)
+    assert (y == 0).all()
+    small = -(-_int8(qt, k, n) // 256) * 256
+    if split:  # at least the copy: runs of whole tiles need no parts
+        assert asked >= -(-_xh(qt, k, n) // 256) * 256
+    else:  # the int8 GEMM on few row tiles splits K too (at most four ways)
+        slots = 4 * 1024 * -(-n // 16) * -(-rows // 16) + 1024 if qt in (o.Q4_K, o.Q6_K, o.IQ4_XS) else 0
+        assert small <= asked <= small + slots and asked != -(-_xh(qt, k, n) // 256) * 256
+
+
+@pytest.mark.parametrize("qt,rows,k,n,split", [(o.IQ3_S, 512, 512, 300, False), (o.IQ3_S, 4096, 4096, 64, False),
+                                               (o.IQ3_S, 6144, 4096, 64, True), (o.Q4_K, 1024, 1024, 512, False)])
+def test_split_plan_of_the_fp16_small_gemms_types(lib, qt, rows, k, n, split):
+    """The same where the small GEMM reads the fp16 copy too: its workspace is the copy alone."""
+    w = torch.zeros(rows, o.BLOCK_BYTES[qt] * (k // 256), dtype=torch.uint8, device="cuda")
+    y, asked = _asked(lib, qt, w, torch.randn(n, k, device="cuda"), rows)
+    assert (y == 0).all() and (asked > _xh(qt, k, n) if split else asked == -(-_xh(qt, k, n) // 256) * 256)

@@ -64,6 +64,7 @@ bool small_h_supported(int type, bool packed);
 bool small_h_range(int type, int64_t nrows, int64_t n);
 hipError_t launch_gemm_small_h(int type, bool packed, const uint8_t* W, int64_t row_bytes, int nrows, int k,
                                const uint8_t* xh, int n, void* y, int y_dtype, hipStream_t stream);
+double prefill_split_us(int type, bool exact, int64_t nrows, int64_t k, int64_t n);
 double prefill_whole_us(int type, bool exact, int64_t nrows, int64_t k, int64_t n);
 hipError_t launch_gemm_prefill(int type, bool exact, bool split, const uint8_t* W, int64_t row_bytes, int nrows, int k,
                                const uint8_t* xh, int n, void* y, int y_dtype, float* part, uint32_t* cnt,
@@ -270,25 +271,49 @@ bool xxs_packed(int op, int64_t type);
 
 bool small_fp16_shape(int op, int64_t type, int64_t k, int64_t n);
 
-// Whether a product op runs the prefill GEMM (gemm_prefill.hip) where its workspace has room for the split
-// plan: a tile of 128 weight rows decoded once per step for up to 256 columns, work split evenly over the
-// CUs, against the small GEMMs' 16-row tiles that decode the weights again for every 4 column tiles.
-// Measured (us per op, graph replays, prefill / the plan it replaces):
-//   34816 x 5120, M = 65 / 256 / 512: IQ3_S 83 / 145 / 257 against 149 / 234 / 353, IQ4_XS 98 / 175 /
-//   317 against 251 / 393 / 607, Q6_K 94 / 151 / 270 against 322 / 249 / 376, IQ2_S 85 / 134 / 254
-//   against 310 / 640 / 1264; 5120 x 6144, M = 65: IQ3_S 31 against 45, Q6_K 32 against 68.
-// On small weights its fixed cost (the table, the K split's parts) shows: 1024 x 5120 M = 100 / 256 /
-// 512 IQ3_S 22 / 24 / 28 against 19 / 22 / 32, 2048 x 5120 M = 100 / 160 23 / 24 against 19 / 29. So from
-// 65 rows on weights of 16M values or more (64 where the fp16 small GEMM's activation layout, the
-// same, served 64), from 129 from 8M values, else from 257. Q2_K, whose other GEMM is the per-slice one,
-// always (12288 x 5120 M = 24 37 against 71; 1024 x 5120 M = 16 21 against 28), up to the K of which one
-// column tile's copy fits the static scratch.
-bool prefill_route(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
+// The product ops that may run the prefill GEMM (gemm_prefill.hip) by the size that
+// gguf_op_workspace_bytes reports, which has room for its activation copy there: from 65 rows on weights
+// of 16M values or more (64 for IQ3_XXS and where the fp16 small GEMM's activation layout, the same, served
+// 64), from 129 from 8M values, else from 257; Q2_K always, up to the K of which one column tile's copy fits
+// the static scratch.
+bool prefill_rows(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
   if (!op_gemm(op) || !gguf::prefill_supported((int)type, op_packed(op))) return false;
   if (type == gguf::kQ2_K) return gguf::xh_bytes(16, k, (int)type) <= kScratchBytes;  // K <= 199k
   const int64_t values = row * k;
-  const int64_t from = values >= (16 << 20) ? (small_fp16_shape(op, type, k, 64) ? 64 : 65) : values >= (8 << 20) ? 129 : 257;
-  return n >= from;
+  if (values < (16 << 20)) return n >= (values >= (8 << 20) ? 129 : 257);
+  return n >= (type == kIQ3_XXS || small_fp16_shape(op, type, k, 64) ? 64 : 65);
+}
+
+bool q6k_rounded(int64_t type, int64_t row, int64_t n);
+double small_us(int64_t type, int64_t row, int64_t k, int64_t n);
+
+// Whether one of them is the faster on the prefill GEMM where the workspace has room for the split plan: a
+// tile of 128 weight rows decoded once per step for up to 256 columns, work split evenly over the CUs,
+// against the small GEMMs' 16-row tiles that decode the weights again for every 4 column tiles. Measured
+// (us per op, graph replays, prefill / the plan it replaces):
+//   34816 x 5120, M = 65 / 256 / 512: IQ3_S 83 / 145 / 257 against 149 / 234 / 353, IQ4_XS 98 / 175 /
+//   317 against 251 / 393 / 607, Q6_K 94 / 151 / 270 against 322 / 249 / 376, IQ2_S 85 / 134 / 254
+//   against 310 / 640 / 1264; 5120 x 6144, M = 65: IQ3_S 33 against 45, Q6_K 38 against 67.
+// It costs about 14 us at K = 512 and 18 to 28 where it adds parts, however small the product, so:
+//  * weights of fewer than 8M values by the estimates of both plans, 1 us apart (within 1 % of the better
+//    one on average over 8 shapes): 512 x 512 M = 257 / 1024 IQ3_S 14 / 15 against 9 / 12, IQ2_S 14 / 15
+//    against 11 / 18; 1024 x 1024 M = 257 / 1024 18 / 20 against 13 / 23, 19 / 20 against 17 / 33; 1024 x 2048 M =
+//    257 / 1024 IQ3_S 22 / 25 against 16 / 32;
+//  * K > 8192 on few rows, where the int8 GEMM of Q4_K, IQ4_XS and Q6_K splits K as well and the prefill
+//    GEMM adds up to 17 parts a tile: IQ4_XS 1024 x 17408 M = 65 / 129 39 / 43 against 31 / 53, 2048 x 17408 M
+//    = 100 / 129 52 / 61 against 45 / 75, 512 x 17408 M = 160 / 512 / 1024 37 / 59 / 75 against 34 / 50 / 91;
+//  * 64 rows of the fp16 small GEMM's types from 24M values: 4096 x 4096 IQ3_S 23 against 18;
+//  * Q2_K, whose other GEMM is the per-slice one, by that one's estimate: M = 16 / 32 / 48 on 1024 x 1024 22 /
+//    23 / 23 against 11 / 14 / 18, 1024 x 2048 24 / 25 / 25 against 15 / 22 / 28, 12288 x 5120 44 / 45 / 45 against
+//    51 / 71 / 98.
+bool split_route(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
+  if (!prefill_rows(op, type, row, k, n)) return false;
+  if (type == gguf::kQ2_K) return small_us(type, row, k, n) > (k <= 512 ? 16 : k <= 1024 ? 22.5 : 25);
+  const int64_t values = row * k;
+  if (values < (8 << 20))
+    return gguf::prefill_split_us((int)type, !q6k_rounded(type, row, n), row, k, n) + 1 < small_us(type, row, k, n);
+  if (k > 8192 && row <= 2048 && !op_packed(op) && !generic(type)) return n >= (row <= 512 ? 1024 : 129);
+  return n >= 65 || type == kIQ3_XXS || values >= (24 << 20);
 }
 
 // Q6_K products with the sub-scale folded into the fp16 operand, rounded beyond 2048 (xh_decode.h): from
@@ -300,13 +325,22 @@ bool q6k_rounded(int64_t type, int64_t row, int64_t n) {
 
 // Estimated time of the small GEMM that a product runs without the prefill GEMM, us: K blocks x workgroups
 // (a 16-row tile and up to four column tiles) per CU x a block's time in one. Q2_K's per-slice GEMM: a
-// workgroup alone on its CU takes 1.6 times that. Fitted like pf_whole_shape's.
+// workgroup alone on its CU takes about 1.6 times that. Fitted like pf_whole_shape's.
 double small_us(int64_t type, int64_t row, int64_t k, int64_t n) {
   const int64_t nct = (n + 15) / 16, nb = k / 256;
   const double tiles = (double)((row + 15) / 16) / 256;
   if (type == gguf::kQ2_K) {
+    const double t = (double)std::min<int64_t>(nct, 4);
     const double wgs = std::ceil(tiles * std::max(1.0, (double)nct / 4));
-    return 12 + (double)nb * (0.35 + 0.33 * (double)std::min<int64_t>(nct, 4)) * std::max(1.6, wgs);
+    return 7 + (double)nb * std::max(1.6 * (0.2 + 0.47 * t), wgs * (0.35 + 0.33 * t));
+  }
+  if (row * k < (8 << 20)) {  // few workgroups: whole rounds of them over the CUs
+    double a = 5, b = 4.2, c = 0.78;
+    if (type == gguf::kIQ3_S) a = 6, b = 2, c = 0.52;
+    if (type == gguf::kQ4_K) a = 6, b = 2.4, c = 0.60;
+    if (type == gguf::kIQ4_XS) b = 4, c = 0.62;
+    if (type == gguf::kIQ2_XXS) c = 0.65;
+    return a + std::ceil(tiles * (double)((nct + 3) / 4)) * (b + c * (double)nb);
   }
   const bool deep = k > 8192;  // IQ3_S and Q4_K run the int8 GEMM instead of the fp16 one
   double per = deep ? 0.78 : 0.76;  // IQ3_XXS, IQ2_S, IQ2_XS
@@ -318,7 +352,7 @@ double small_us(int64_t type, int64_t row, int64_t k, int64_t n) {
   return 12 + (double)nb * per * tiles * (double)((nct + 3) / 4);
 }
 
-// Whether a product of prefill_route runs the prefill GEMM without room for the split plan's parts, in
+// Whether a product of prefill_rows runs the prefill GEMM without room for the split plan's parts, in
 // whole tiles: a tile walks all of K, so on a grid of few tiles most CUs idle, and the small GEMMs, whose
 // 16-row tiles spread the same work, are the faster ones. By the estimates of both. Measured, us, whole
 // tiles (their best width) / small GEMM / split plan: 5120 x 17408 M = 100 IQ3_S 140 / 132 / 63, Q2_K 226 /
@@ -328,24 +362,30 @@ double small_us(int64_t type, int64_t row, int64_t k, int64_t n) {
 // 18 % (IQ3_S 34816 x 5120 M = 160 194 against 164), and at worst 4 % slower than the GEMM that ran before
 // the split plan took the product over.
 bool whole_route(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
-  return prefill_route(op, type, row, k, n) &&
+  return prefill_rows(op, type, row, k, n) &&
          gguf::prefill_whole_us((int)type, !q6k_rounded(type, row, n), row, k, n) < small_us(type, row, k, n);
 }
 
-// Where the prefill GEMM is the faster one below those rows, but its activation copy is twice the
+// Where the split plan is the faster one below those rows, but its activation copy is twice the
 // int8 layouts': taken when the library sizes the workspace itself (gguf_mul_mat_alloc), so that the
 // size that gguf_op_workspace_bytes reports stays the smaller one. From 33 rows on weights of 24M
 // values or more (M = 48: Q6_K 5120 x 6144 25 against 33 us, 34816 x 5120 76 against 135; Q4_K 73
-// against 111; IQ2_S 17408 x 5120 41 against 53), packed IQ3_S there from 80M values (34816 x 5120 64
-// against 80, 5120 x 17408 45 against 49; 8192 x 5120 25 against 24) and everything from 49 rows (M =
-// 56: IQ3_S 8192 x 5120 25 against 37); not where the fp16 range plan applies (17408 x 5120 M = 48
-// IQ3_S 42 against 41, Q4_K 45 against 40).
-bool prefill_preferred(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
-  if (prefill_route(op, type, row, k, n)) return true;
-  if (!op_gemm(op) || !gguf::prefill_supported((int)type, op_packed(op))) return false;
+// against 111; IQ2_S 17408 x 5120 41 against 53), there packed IQ3_S from 80M values (34816 x 5120 64
+// against 80, 5120 x 17408 45 against 49; 8192 x 5120 25 against 24), IQ3_XXS and IQ2_XXS from 48M (8192 x
+// 5120 25 against 23, 25 against 22), IQ4_XS with K > 8192 from 64M (3072 x 17408 40 against 34), and
+// everything from 49 rows (M = 56: IQ3_S 8192 x 5120 25 against 37; M = 49 IQ4_XS 3072 x 17408 41 against 51);
+// not where the fp16 range plan applies (17408 x 5120 M = 48 IQ3_S 42 against 41, Q4_K 45 against 40), nor
+// where split_route leaves more rows to the int8 GEMM.
+bool split_preferred(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
+  if (prefill_rows(op, type, row, k, n) || !op_gemm(op) || !gguf::prefill_supported((int)type, op_packed(op)))
+    return split_route(op, type, row, k, n);
   if (small_fp16_shape(op, type, k, n) && gguf::small_h_range((int)type, row, n)) return false;
-  const int64_t values = row * k;
-  return (n >= 33 && values >= (type == gguf::kIQ3_S ? (80 << 20) : (24 << 20))) || (n >= 49 && values >= (24 << 20));
+  if (k > 8192 && row <= 2048 && !op_packed(op) && !generic(type)) return false;
+  const int64_t from = type == gguf::kIQ3_S                              ? 80
+                       : type == kIQ3_XXS || type == gguf::kIQ2_XXS      ? 48
+                       : type == gguf::kIQ4_XS && k > 8192               ? 64
+                                                                         : 24;
+  return row * k >= (n >= 49 ? 24 << 20 : n >= 33 ? from << 20 : INT64_MAX);
 }
 
 int64_t vec_mma_from(int op, int64_t type) {
@@ -472,8 +512,8 @@ enum class Plan { kSmall, kWhole, kSplit };
 // The plan of a workspace of `bytes` bytes: the fastest one that fits it (kSmall, which may not fit either,
 // if none does).
 Plan plan_for(int op, int64_t type, int64_t row, int64_t k, int64_t n, size_t bytes) {
-  if (!prefill_route(op, type, row, k, n) || bytes < prefill_ws(type, k, n)) return Plan::kSmall;
-  if (bytes >= prefill_split_ws(type, row, k, n)) return Plan::kSplit;
+  if (!prefill_rows(op, type, row, k, n) || bytes < prefill_ws(type, k, n)) return Plan::kSmall;
+  if (split_route(op, type, row, k, n) && bytes >= prefill_split_ws(type, row, k, n)) return Plan::kSplit;
   return whole_route(op, type, row, k, n) ? Plan::kWhole : Plan::kSmall;
 }
 
@@ -483,7 +523,7 @@ Plan plan_for(int op, int64_t type, int64_t row, int64_t k, int64_t n, size_t by
 size_t gguf_op_workspace_bytes(int op, int64_t type, int64_t row, int64_t k, int64_t n, int has_x_q8) {
   if (n <= 0) return 0;
   const size_t small = small_ws(op, type, row, k, n, has_x_q8 != 0);
-  return prefill_route(op, type, row, k, n) ? std::max(small, prefill_ws(type, k, n)) : small;
+  return prefill_rows(op, type, row, k, n) ? std::max(small, prefill_ws(type, k, n)) : small;
 }
 
 }  // extern "C"
@@ -686,7 +726,7 @@ int gguf_mul_mat_alloc(int op, const gguf_view* W, const gguf_view* X, int64_t t
   if (n == 0) return GGUF_OK;
   const DeviceScope scope(X->device);
   if (scope.err != hipSuccess) return hip_fail(scope.err, name, "device select");
-  const Plan plan = prefill_preferred(op, type, row, k, n) ? Plan::kSplit : Plan::kSmall;
+  const Plan plan = split_preferred(op, type, row, k, n) ? Plan::kSplit : Plan::kSmall;
   const size_t need = plan == Plan::kSplit ? prefill_split_ws(type, row, k, n)
                                            : small_ws(op, type, row, k, n, x_q8 != nullptr);
   void* ws = nullptr;
@@ -715,7 +755,7 @@ bool noalloc_beyond_scratch(int op, int64_t type, int64_t row, int64_t k, int64_
   const bool fp16 = xxs_packed(op, type) ? (n >= 256 && groups >= 32) || (n >= 64 && groups >= 128)
                     : type == gguf::kIQ3_S || type == gguf::kQ4_K || type == gguf::kQ6_K ? n >= 256 && groups >= 64
                                                                                          : false;
-  return prefill_route(op, type, row, k, n) && !fp16 && small_ws(op, type, row, k, n, false) <= kScratchBytes;
+  return prefill_rows(op, type, row, k, n) && !fp16 && small_ws(op, type, row, k, n, false) <= kScratchBytes;
 }
 
 void* g_scratch_ptr[gguf::kMaxDevices] = {};

@@ -494,7 +494,7 @@ struct PfShape {
 // 133 / 89 / 115, M = 512 271 / 305 / 400. For the other types it takes the fastest rs as well, within 1 %
 // on average over 12 shapes and 14 row counts each, at worst 19 % (6144 x 2048 M = 300 IQ4_XS, 40 us at rs = 2
 // against 33 at 4).
-PfShape pf_shape(int64_t nrows, int64_t k, int64_t n) {
+PfShape pf_shape(int64_t nrows, int64_t k, int64_t n, double* us = nullptr) {
   static const double fixed[3] = {20, 16, 14}, few[3] = {3.5, 2.3, 1.7}, full[3] = {5.6, 3.0, 2.3};
   const int64_t nct = xq_col_tiles(n), nb = k / kQK, nrg = (nrows + 127) / 128, cus = device_cus();
   PfShape best{1, 0, 0};
@@ -506,6 +506,7 @@ PfShape pf_shape(int64_t nrows, int64_t k, int64_t n) {
     const double t = fixed[i] + (double)((units + wgs - 1) / wgs) * (few[i] + (full[i] - few[i]) * (double)wgs / (double)cus);
     if (i == 0 || t < least) least = t, best = {rs, tiles, wgs};
   }
+  if (us) *us = least;
   return best;
 }
 
@@ -574,11 +575,18 @@ size_t prefill_slot_bytes(int64_t nrows, int64_t k, int64_t n) {
   return (size_t)(s.wgs + std::min(s.wgs, s.tiles)) * (16 / s.rs) * 2 * 4096;
 }
 
-// Estimated time of a product in whole tiles, us.
+// Estimated time of a product with K split over the CUs, us: pf_shape's, less on the shortest K
+// (fewer parts or none), more where Q6_K's operands take two planes.
+double prefill_split_us(int type, bool exact, int64_t nrows, int64_t k, int64_t n) {
+  double us = 0;
+  (void)pf_shape(nrows, k, n, &us);
+  return us - (k <= 512 ? 7 : k <= 1024 ? 2.5 : 0) + (type == kQ6_K && exact ? 2.5 : 0);
+}
+// Estimated time of a product in whole tiles, us (512 x 512 M = 257 14, 1024 x 1024 18.6).
 double prefill_whole_us(int type, bool exact, int64_t nrows, int64_t k, int64_t n) {
   double us = 0;
-  pf_whole_shape(type, exact, nrows, k, n, &us);
-  return us;
+  (void)pf_whole_shape(type, exact, nrows, k, n, &us);
+  return us + (k <= 1024 ? 2 : 0);
 }
 
 // Large-M products; xh: X in the xh layout of the type. split: K over the CUs, with prefill_slot_bytes of
