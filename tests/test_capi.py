@@ -58,7 +58,7 @@ def test_workspace_follows_the_product_plan(lib):
     layout (4,608 B per 16 rows x 256 values) below 64 rows, the fp16 one (9,216 B) for packed
     IQ3_S and Q4_K from 64 rows at K <= 8192, below that where the fp16 GEMM's range plan takes
     the weight (1..5 row tiles per CU, 256 CUs assumed without a GPU; IQ3_S from 33 rows, Q4_K
-    from 17), and for the prefill from 256 rows; IQ4_XS and K = 17408 stay on the int8 layout below the prefill
+    from 17), and wherever the prefill GEMM may run; IQ4_XS and K = 17408 stay on the int8 layout at 64 rows
     (plus a K split's slots and counters on grids of few tiles)."""
     xq = lambda n, k: -(-n // 16) * (k // 256) * 4608
     xh = lambda n, k: -(-n // 16) * (k // 256) * 9216

@@ -48,7 +48,7 @@ CASES = [
     (o.Q4_K, 5120, 17408, 16, False),   # int8 raw GEMM with K split
     (o.Q4_K, 4096, 5120, 1, False),     # row-chunk GEMV
     (o.Q6_K, 1024, 5120, 4, False),     # raw GEMV
-    (o.IQ4_XS, 1024, 5120, 512, False), # int8 prefill GEMM
+    (o.IQ4_XS, 1024, 5120, 512, False), # fp16 prefill GEMM, K split over workgroups
     (o.IQ2_S, 1024, 5120, 2, False),    # generic GEMV
     (o.IQ2_S, 1024, 5120, 16, False),   # generic MFMA GEMM
     (o.IQ3_S, 1024, 5120, 16, False),   # per-slice MFMA GEMM (unpacked IQ3_S)

@@ -321,8 +321,9 @@ def test_golden_rows(qt, n):
 
 
 # ------------------------------------------------------------------------------------ fp16 small GEMM
-# Product ops of 64..255 activation rows with K <= 8192 on packed IQ3_S and Q4_K run the fp16
-# small GEMM: one 16-row tile per workgroup below 1024 tiles, two from 1024 tiles on.
+# Packed IQ3_S and Q4_K with K <= 8192 run the fp16 small GEMM from 64 activation rows where the prefill
+# GEMM is not the faster one: one 16-row tile per workgroup below 1024 tiles, two from 1024 tiles on. (The
+# larger size runs the prefill GEMM at 255 rows of K = 512, and at K = 2048.)
 SMALL_H_ROWS = {o.IQ3_S: (64, 16 * 1025), o.Q4_K: (100, 16 * 1024 + 9)}
 
 
@@ -542,7 +543,8 @@ def test_packed_ops_vs_q81(n, k):
 
 
 # ------------------------------------------------------------------------------------ prefill
-# Product ops from 256 activation rows on run the 128 x 128-tile prefill GEMM.
+# Product ops of many activation rows: the prefill GEMM or, on the smallest weights here, the small GEMMs,
+# whichever is estimated faster (test_gpu_prefill_plans.py pins each plan of the prefill GEMM).
 PREFILL_N = [256, 300, 600]
 
 
@@ -567,7 +569,7 @@ def test_prefill_exact_integer_dots(qt, n):
 
 @pytest.mark.parametrize("qt", TYPES, ids=lambda t: TN[t])
 def test_prefill_wide_exact_integer_dots(qt):
-    """A grid of 256 workgroup tiles (the prefill GEMM's wide-workgroup plan for IQ3_S / Q4_K),
+    """4096 x 512 with 2048 activation rows (128-column tiles of the prefill GEMM),
     in the exact-integer mode; with every scale 1 the float64 q81 model is the exact integer."""
     from vllm_gguf_plugin.quantization import iq3_pack
 
@@ -596,8 +598,8 @@ def test_prefill_vs_q81(qt, n):
 
 
 def test_prefill_q6k_largest_subscales():
-    """Q6_K on the fp16 prefill GEMM folds each 16-value sub-scale into the decoded operand;
-    (q - 32) * sc is exact in fp16 up to 2048 and rounds beyond. Every sub-scale at +-127 (each
+    """Q6_K at 300 rows of a small weight (the int8 GEMM; the prefill GEMM's rounded operands, (q - 32) * sc
+    beyond 2048, and its exact ones: test_gpu_prefill_plans.py). Every sub-scale at +-127 (each
     product of magnitude 2048..4064 then rounds): the output still meets the fp32 bar of the
     float64 model, and an exact-integer run with sub-scales in [-64, 64] (odd products up to
     2047 in magnitude, all exact) matches the integer sum."""
@@ -621,7 +623,7 @@ def test_prefill_q6k_largest_subscales():
 @pytest.mark.parametrize("n", PREFILL_N)
 @pytest.mark.parametrize("k", [512, 1536])
 def test_prefill_packed_xxs_exact(n, k):
-    """IQ3_XXS in its unit layout on the fp16 prefill GEMM (operand w * ls, row scale d / 4), in
+    """IQ3_XXS in its unit layout at the prefill GEMM's row counts (on this weight the generic GEMM), in
     the exact mode: the product ops' slice values dot / 4 summed, multiples of 1/4 exact in fp32;
     144 rows (a partial last 128-row group) and K = 1536 (a ragged last unit-block)."""
     from vllm_gguf_plugin.quantization import iq3_pack
@@ -637,7 +639,7 @@ def test_prefill_packed_xxs_exact(n, k):
 
 @pytest.mark.parametrize("rows,k,n", [(272, 5120, 256), (272, 5120, 600), (2048, 5120, 2048)])
 def test_prefill_packed_xxs_vs_q81(rows, k, n):
-    """IQ3_XXS prefill (the 4-wave and the 8-wave plans) against the q81 model of the product ops."""
+    """IQ3_XXS products of many rows (the generic GEMM, the prefill GEMM) against the q81 model."""
     from vllm_gguf_plugin.quantization import iq3_pack
 
     raw = _w(o.IQ3_XXS, rows, k, seed=rows + n + 9)

@@ -1,9 +1,8 @@
-"""The prefill GEMM's plans at their edges, in the exact-integer mode (every scale 1, so that any order
-of the sums gives the same output): K split over workgroups (the torch ops, whose workspace has room
-for the parts) and unsplit (gguf_mul_mat with the workspace gguf_op_workspace_bytes asks for), for
-every type it serves, at row counts that are no multiple of a 128-row tile and activation rows at the
-edges of its 64-, 128- and 256-column tiles; graph replays of a split product; Q6_K's two-plane
-operands at the largest sub-scales; the no-allocation entry point in parts. Needs an MI355X.
+"""Product ops around the prefill GEMM's plans: which one runs (the split over K, whole tiles, the small
+GEMMs) by the workspace that is asked for or written, with the workspace of the reported size, less, and
+none (the no-allocation entry point); the small shapes on which all of them meet, in the exact-integer
+mode; Q2_K's rounded scales, group sums and mins beyond fp16. Each plan and tile width of the prefill GEMM:
+test_gpu_prefill_plans.py. Needs an MI355X.
 """
 
 import ctypes
@@ -59,8 +58,8 @@ def _capi_op(lib, qt, w, x, rows, entry="workspace"):
     return y, nb
 
 
-# rows (packed types: the next multiple of 16), K, activation rows: two row tiles and a ragged third, K
-# blocks that the runs cut unevenly; one 16-row tile; K of one step pair
+# rows (packed types: the next multiple of 16), K, activation rows: small weights, of which the small GEMMs
+# run most
 SHAPES = [(270, 4608, 257), (270, 4608, 300), (16, 1024, 513), (1030, 512, 259), (130, 2560, 1025)]
 
 
@@ -91,8 +90,8 @@ def test_q2k_every_row_count(n):
 @pytest.mark.parametrize("qt", [o.Q4_K, o.IQ4_XS, o.Q6_K, o.IQ2_S], ids=lambda t: o.TYPE_NAMES[t])
 @pytest.mark.parametrize("n", [33, 49, 64])
 def test_rows_33_to_64(qt, n):
-    """Weights of 24M values or more at 33..64 rows: the torch ops prefer the prefill GEMM there (64
-    columns per workgroup, K split). fp32 X against the q81 model on sampled rows."""
+    """Weights of 24M values or more at 33..64 rows: the torch ops prefer the prefill GEMM there (K split;
+    asserted in test_gpu_prefill_plans.py). fp32 X against the q81 model on sampled rows."""
     rows, k = 5120, 5120
     raw = w_rand(qt, rows, k, seed=n)
     x = x_rand(n, k, seed=n + 7)
@@ -102,8 +101,8 @@ def test_rows_33_to_64(qt, n):
 
 
 def test_split_graph_replays():
-    """Replays of a captured split product (its counters are cleared by the captured quantise launch),
-    with eager work between, equal the eager result bit for bit."""
+    """Replays of a captured product, with eager work between, equal the eager result bit for bit (the
+    prefill GEMM's split plan: test_split_replays)."""
     raw = w_rand(o.Q4_K, 1030, 2560, seed=1)
     w, x = dev(raw), x_rand(300, 2560, seed=2, dtype=torch.bfloat16).cuda()
     eager = _torch_op(o.Q4_K, w, x, 1030)
@@ -112,8 +111,8 @@ def test_split_graph_replays():
 
 
 def test_q6k_two_planes_largest_subscales():
-    """Q6_K below the rounded plan's rows: every sub-scale +-127 or -128, products up to 4096 kept
-    exact in two operand planes (the int8 GEMM's results)."""
+    """Q6_K below the rounded plan's rows: every sub-scale +-127 or -128, products up to 4096 kept exact
+    (the int8 GEMM; the prefill GEMM's two operand planes: test_q6k_two_planes_on_the_split_plan)."""
     rows, k, n = 270, 2560, 259
     raw = exact_weights(o.Q6_K, rows, k, seed=3)
     sc = np.random.default_rng(4).choice(np.array([127, -127, -128], np.int8), size=(rows * k // 256, 16))
@@ -128,7 +127,8 @@ def test_q6k_two_planes_largest_subscales():
 @pytest.mark.parametrize("qt,n", [(o.IQ4_XS, 1100), (o.IQ2_S, 1100), (o.Q2_K, 900)], ids=["IQ4_XS", "IQ2_S", "Q2_K"])
 def test_noalloc_in_parts(lib, qt, n):
     """Products whose fp16 activation copy exceeds the static scratch and whose int8 copy fits it: the
-    no-allocation entry point runs them in parts of the activation rows, with the same results."""
+    no-allocation entry point runs them on the latter (in parts on larger weights, test_x_view_in_parts),
+    with the same results."""
     rows, k = 400, 5120
     w = dev(w_rand(qt, rows, k, seed=n))
     x = x_rand(n, k, seed=n + 1, dtype=torch.float32).cuda()
@@ -199,7 +199,7 @@ def test_q2k_min_beyond_fp16(n, group):
     q, _ = o.dequant_q8_1_mmq(q8, n, k, o.Q2_K)
     sums = o.mmq_d2s6_sums(q8, n, k).reshape(n, k // 16)
     sums = np.where(np.isnan(sums), q.astype(np.int64).reshape(n, k // 16, 16).sum(-1), sums)[:, 16 + group]
-    want = np.where(sums == 0, np.nan, -np.sign(sums) * np.inf).astype(np.float32)
+    want = np.where(sums == 0, np.nan, np.where(sums < 0, np.inf, -np.inf)).astype(np.float32)
     assert (sums > 0).any() and (sums < 0).any()
     assert np.array_equal(y[:, bad], np.repeat(want[:, None], len(bad), 1), equal_nan=True)
     assert np.isfinite(np.delete(y, bad, axis=1)).all()

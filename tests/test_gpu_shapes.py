@@ -233,7 +233,7 @@ def _residual_heavy_x(n, k, seed):
                                   ("lcpp_mul_mat_vec_q", 1)])
 def test_q4k_min_term_form(op, n):
     """Q4_K on activations whose slice sums differ from d * sum(q) by about 10 %: the product ops
-    (int8 small GEMM, fp16 small GEMM at 64-255 rows, prefill from 256 rows) follow the MMQ form
+    (int8 small GEMM, fp16 small GEMM, prefill GEMM) follow the MMQ form
     dmin * m * half(sum x), the decode ops (GEMV, and the int8 GEMM they take from 3 rows) the
     MMVQ form dmin * m * d8 * sum(q8); the two forms are more than 1e-2 apart here."""
     rows, k = 2304 if op == "lcpp_mul_mat_vec_own" else 272, 2048

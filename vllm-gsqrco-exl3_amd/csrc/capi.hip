@@ -316,7 +316,7 @@ bool split_route(int op, int64_t type, int64_t row, int64_t k, int64_t n) {
   return n >= 65 || type == kIQ3_XXS || values >= (24 << 20);
 }
 
-// Q6_K products with the sub-scale folded into the fp16 operand, rounded beyond 2048 (xh_decode.h): from
+// Q6_K products with the sub-scale folded into the fp16 operand, rounded beyond 2048 (pf_decode.h): from
 // 256 rows on grids of 64 tiles of 128 x 256 or more. Elsewhere its operands are exact, as the int8
 // GEMM's are: two MFMAs per slice instead of one.
 bool q6k_rounded(int64_t type, int64_t row, int64_t n) {

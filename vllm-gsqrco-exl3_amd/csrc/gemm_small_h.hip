@@ -1,6 +1,6 @@
 // Small-batch GEMM on fp16 MFMA for IQ3_S (tile layout) and Q4_K rows: Y[c, r] = sum_k X[c, k] *
-// W[r, k] for product ops below the prefill GEMM's rows: from 64 activation rows on small weights, and
-// the range plan's 17..48.
+// W[r, k] for product ops with K <= 8192 off the prefill GEMM: from 64 activation rows on weights too small
+// for it or without the workspace of its split plan, and the range plan's 17..48.
 //
 // Replaces the reference's tiled products at these row counts (lcpp_owned_iq3_mma.cu:614-1096 for
 // packed IQ3_S, vendored MMQ for Q4_K) with a gfx950 design on the exact fp16 route of the prefill
@@ -8,8 +8,8 @@
 // v_mfma_f32_16x16x32_f16 returns sub-scale x integer slice dot exactly in fp32 and the per-slice
 // epilogue is one FMA by the activation scale (the int8-MFMA route needs an integer multiply, a
 // conversion and an FMA per output element and slice).
-//  * A workgroup owns RT (1 or 2) 16-row tiles and NM (1, 2 or 4) column tiles of 16 activation
-//    rows (grid y walks groups of NM column tiles). Its 2 RT decoder waves and NM multiplier waves
+//  * A workgroup owns RT (1 or 2; the range plan 5) 16-row tiles and NM (4; the range plan 2 or 3) column
+//    tiles of 16 activation rows (grid y walks groups of NM column tiles). Its 2 RT decoder waves and NM multiplier waves
 //    work on consecutive K blocks: while the multipliers use block b from one LDS A area, decoder
 //    w writes half block w & 1 of row tile w >> 1 of block b + 1 into the other (one row slice of
 //    32 values per lane), with one LDS-only barrier per block. Each role runs its own loop, so no
@@ -41,8 +41,8 @@ constexpr Iq3sSignedTable make_iq3s_biased_table() {
 }
 __device__ const Iq3sSignedTable kIq3sBiased = make_iq3s_biased_table();
 
-// decode_step for IQ3_S (same lane mapping, A layout and block-scale handling) through the
-// biased table in LDS (tbl)
+// The lane's slice of row j, IQ3_S, through the biased table in LDS (tbl): the A layout and the running
+// block scale are those of Q4_K's decode_step (xh_decode.h)
 __device__ __forceinline__ void decode_step_tb(const RawIq3& w, int h, const uint8_t* tbl, uint8_t* A, float* RT,
                                                float* EF, float& e, int t, int j, int sp) {
   const int s = 4 * h + sp;
@@ -336,11 +336,8 @@ void launch_small_h_t(const uint8_t* W, int64_t row_bytes, int nrows, int k, con
 template <int TYPE, int RT>
 void launch_small_h_rt(const uint8_t* W, int64_t row_bytes, int nrows, int k, const uint8_t* xh, int n, void* y,
                        int y_dtype, hipStream_t stream) {
-  const int nct = (int)xq_col_tiles(n);
   const unsigned gx = (unsigned)(((nrows + 15) / 16 + RT - 1) / RT);
-  if (nct <= 1) launch_small_h_t<TYPE, RT, 1, 2, false>(W, row_bytes, nrows, k, xh, n, y, y_dtype, gx, stream);
-  else if (nct <= 2) launch_small_h_t<TYPE, RT, 2, 2, false>(W, row_bytes, nrows, k, xh, n, y, y_dtype, gx, stream);
-  else launch_small_h_t<TYPE, RT, 4, 2, false>(W, row_bytes, nrows, k, xh, n, y, y_dtype, gx, stream);
+  launch_small_h_t<TYPE, RT, 4, 2, false>(W, row_bytes, nrows, k, xh, n, y, y_dtype, gx, stream);
 }
 
 // one workgroup per CU over at most kRangeTiles row tiles each, 1..3 column tiles
@@ -364,9 +361,9 @@ bool small_h_range(int type, int64_t nrows, int64_t n) {
   return n >= from && n <= 3 * 16 && tiles >= 4 * cus && tiles <= kRangeTiles * cus;
 }
 
-// xh: X in the xh layout (launch_quantize_xh / launch_q8_1_to_xh). The range plan where it
-// applies; else two row tiles per workgroup from 1024 tiles on (X read once per tile pair), one
-// below (more workgroups on smaller weights).
+// xh: X in the xh layout (launch_quantize_xh). The range plan where it applies; else (64 rows or more)
+// two row tiles per workgroup from 1024 tiles on (X read once per tile pair: 16384 x 512 M = 65 / 128 18.5 /
+// 20.3 us against 27.2 / 29.0 with one), one below (more workgroups on smaller weights).
 hipError_t launch_gemm_small_h(int type, bool packed, const uint8_t* W, int64_t row_bytes, int nrows, int k,
                                const uint8_t* xh, int n, void* y, int y_dtype, hipStream_t stream) {
   if (!small_h_supported(type, packed)) return hipErrorInvalidValue;
