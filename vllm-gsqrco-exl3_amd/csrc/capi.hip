@@ -291,9 +291,9 @@ double small_us(int64_t type, int64_t row, int64_t k, int64_t n);
 // tile of 128 weight rows decoded once per step for up to 256 columns, work split evenly over the CUs,
 // against the small GEMMs' 16-row tiles that decode the weights again for every 4 column tiles. Measured
 // (us per op, graph replays, prefill / the plan it replaces):
-//   34816 x 5120, M = 65 / 256 / 512: IQ3_S 83 / 145 / 257 against 149 / 234 / 353, IQ4_XS 98 / 175 /
-//   317 against 251 / 393 / 607, Q6_K 94 / 151 / 270 against 322 / 249 / 376, IQ2_S 85 / 134 / 254
-//   against 310 / 640 / 1264; 5120 x 6144, M = 65: IQ3_S 33 against 45, Q6_K 38 against 67.
+//   34816 x 5120, M = 65 / 256 / 512: IQ3_S 85 / 135 / 254 against 143 / 234 / 351, IQ4_XS 95 / 167 /
+//   313 against 248 / 388 / 601, Q6_K 118 / 134 / 244 against 311 / 250 / 371, IQ2_S 82 / 130 / 250
+//   against 305 / 635 / 1257; 5120 x 6144, M = 65: IQ3_S 33 against 45, Q6_K 38 against 67.
 // It costs about 14 us at K = 512 and 18 to 28 where it adds parts, however small the product, so:
 //  * weights of fewer than 8M values by the estimates of both plans, 1 us apart (within 1 % of the better
 //    one on average over 8 shapes): 512 x 512 M = 257 / 1024 IQ3_S 14 / 15 against 9 / 12, IQ2_S 14 / 15

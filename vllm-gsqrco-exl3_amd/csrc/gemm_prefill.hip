@@ -490,8 +490,8 @@ struct PfShape {
 // fixed(rs) + blocks per workgroup x block(rs), a block's time growing with the workgroups at work.
 // IQ3_S, K = 5120, slopes and intercepts over rows and K splits: block 3.5 / 2.3 / 1.7 us with a few
 // workgroups and 5.6 / 3.0 / 2.3 with 256 for rs = 1 / 2 / 4, fixed 20 / 16 / 14. Measured at rs =
-// 1 / 2 / 4: 1024 rows M = 256 48 / 32 / 25 us, 8192 rows M = 128 49 / 33 / 34, 34816 rows M = 100
-// 133 / 89 / 115, M = 512 271 / 305 / 400. For the other types it takes the fastest rs as well, within 1 %
+// 1 / 2 / 4: 1024 rows M = 256 47 / 32 / 25 us, 8192 rows M = 128 51 / 36 / 36, 34816 rows M = 100
+// 130 / 86 / 111, M = 512 254 / 304 / 415. For the other types it takes the fastest rs as well, within 1 %
 // on average over 12 shapes and 14 row counts each, at worst 19 % (6144 x 2048 M = 300 IQ4_XS, 40 us at rs = 2
 // against 33 at 4).
 PfShape pf_shape(int64_t nrows, int64_t k, int64_t n, double* us = nullptr) {
